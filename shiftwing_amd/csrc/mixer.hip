@@ -8,19 +8,20 @@
 // (the reference's GPU path rounds them to fp16 first); outputs agree with
 // the CPU path within 1e-3 x RMS.
 //
-// Gated DeltaNet step, three launches:
-//   k_mix_proj<4,..,CONV>  qkv and z projections of every token in one grid;
-//                          a wave that owns a qkv channel also runs that
-//                          channel's causal convolution ring for the tokens in
-//                          order (write the new raw value, SiLU of the tap sum),
-//                          so the ring never crosses workgroups;
-//   k_gdn_recur            one workgroup per (value head, slot group): the
-//                          head's dk x dv state lives in registers (lane halves
-//                          split the key index, 64 values a lane) for all of the
-//                          group's tokens, read and written once per call;
-//   k_mix_proj<4>          the out projection.
-// GQA attention step, five launches:
-//   k_mix_proj<4>          q (query | gate per head), k and v projections;
+// Gated DeltaNet step:
+//   projections            qkv and z of every token in one grid; whoever finishes
+//                          a qkv channel also runs that channel's causal
+//                          convolution ring for the call's tokens (write the new
+//                          raw value, SiLU of the tap sum), so the ring never
+//                          crosses workgroups;
+//   k_gdn_recur            one wave per (value head, 32 value columns, slot
+//                          group): its slice of the dk x dv state lives in
+//                          registers (lane halves split the key index, 64 values
+//                          a lane) for all of the group's tokens, read and
+//                          written once per call;
+//   projection             out.
+// GQA attention step:
+//   projections            q (query | gate per head), k and v;
 //   k_gqa_prep             per-head RMS norm (1 + w) and partial rotary
 //                          embedding of q and k, the K/V append;
 //   k_gqa_attn<HD>         flash decoding on the fp32 matrix cores: one wave per
@@ -29,14 +30,16 @@
 //                          v_mfma_f32_16x16x4f32 (the kv head's query heads are
 //                          the 16 MFMA columns), online softmax in between;
 //   k_gqa_combine          merges the splits, divides, applies the sigmoid gate;
-//   k_mix_proj<4|8>        the o projection (int4 groups or int8 rows).
+//   projection             o (int4 groups or int8 rows).
 //
-// The projection kernel is one design for all of them: a workgroup owns 8
-// rows, each wave 2; every lane loads 16 bytes of each row per 64-lane chunk
-// (32 int4 or 16 int8 columns) with one scale, decodes them to fp32 once and
-// applies them to every token of the call (up to 16) staged in LDS
-// conflict-free ([token][float4 k][lane]).  HBM traffic is the weights once
-// per call; activations come from LDS.
+// A projection streams its weights once per 16 tokens.  From two tokens on
+// it runs on the int8 matrix cores (k_mix_digits, k_mix_mfma,
+// sw_mixer_mfma.h); one token takes k_mix_proj_direct, whose fp32 FMAs need
+// no digits launch.  Layouts outside the converter's 128-column groups take
+// k_mix_proj_direct up to four tokens and k_mix_proj above: every lane loads
+// 16 bytes of each of its rows per 64-lane chunk (32 int4 or 16 int8
+// columns), decodes them to fp32 once and applies them to every token staged
+// in LDS ([token][float4 k][lane]).
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <string.h>
@@ -44,6 +47,7 @@
 #include "sw_backend.h"
 #include "sw_device.h"
 #include "sw_lds_dma.h"
+#include "sw_mixer_mfma.h"
 
 namespace sw {
 namespace {
@@ -842,6 +846,12 @@ __global__ __launch_bounds__(256) void k_gqa_combine(CombArgs c) {
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
+// Tokens from which the int8 matrix cores take the projections.  Per call at
+// 1 / 2 / 4 tokens, matrix cores (with the digits launch) against the vector
+// kernels: S397 Gated DeltaNet 39.0 / 39.7 / 42.2 against 34.1 / 48.8 / 75.3 us,
+// S397 GQA 48.7 / 48.6 / 49.4 against 41.7 / 53.3 / 71.7, S35 Gated DeltaNet
+// 27.5 / 27.7 / 28.5 against 22.8 / 28.8 / 40.8.
+constexpr int kMfmaMinTok = 2;
 int tok_bucket(int B) { return B <= 1 ? 1 : B <= 2 ? 2 : B <= 4 ? 4 : B <= 8 ? 8 : 16; }
 
 // A projection layout the kernel takes: 16-byte rows, 32-column groups.
@@ -1083,7 +1093,7 @@ void launch_proj_direct(ColiCuda *ctx, const ProjArgs &a) {
 }
 
 template <int FMT, bool CONV>
-void launch_proj(ColiCuda *ctx, const ProjArgs &a) {
+void launch_proj_vector(ColiCuda *ctx, const ProjArgs &a) {
   switch (tok_bucket(a.B)) {
     case 1: launch_proj_direct<FMT, 1, CONV>(ctx, a); break;
     case 2: launch_proj_direct<FMT, 2, CONV>(ctx, a); break;
@@ -1091,6 +1101,123 @@ void launch_proj(ColiCuda *ctx, const ProjArgs &a) {
     case 8: launch_proj_nt<FMT, 8, CONV>(ctx, a); break;
     default: launch_proj_nt<FMT, 16, CONV>(ctx, a); break;
   }
+}
+
+// The layouts k_mix_mfma takes: whole 128-column groups (the converter's
+// int4 rows, or int8 rows), at most 64 of them, and a convolution of at most
+// four taps.
+template <int FMT, bool CONV>
+bool mfma_takes(const ProjArgs &a) {
+  return a.cols % 128 == 0 && a.cols / 128 <= kMfmaMaxGroups && (FMT == 8 || a.gs == 128) &&
+         (!a.msp || a.hw % 8 == 0) && (!CONV || (a.K <= 4 && a.B <= kDigTile));
+}
+
+template <int FMT, int W, int GW, bool CONV>
+int launch_mfma(ColiCuda *ctx, dim3 grid, const MfmaArgs &f) {
+  const void *fn = (const void *)k_mix_mfma<FMT, W, GW, CONV>;
+  constexpr int lds = MfmaRing<FMT, W, GW, CONV>::lds;
+  const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (e != hipSuccess) return fail_hip("mixer projection attributes", e);
+  k_mix_mfma<FMT, W, GW, CONV><<<grid, 64 * W, lds, ctx->stream>>>(f);
+  return 0;
+}
+
+// Digits of the call's activations (scratch `dig`, mix_digit_bytes), then the
+// weights against them.
+template <int FMT, bool CONV>
+int launch_proj_mfma(ColiCuda *ctx, const ProjArgs &a, unsigned char *dig) {
+  const int tiles = (a.B + kDigTile - 1) / kDigTile;
+  DigitArgs d;
+  memset(&d, 0, sizeof(d));
+  d.x = a.x;
+  d.ldx = a.ldx;
+  d.cols = a.cols;
+  d.T = a.B;
+  d.dig = dig;
+  d.asc = (float *)(dig + mix_digit_scales_at(a.B, a.cols));
+  d.msp = a.msp;
+  d.nsp = a.nsp;
+  d.hw = a.hw;
+  d.eps = a.eps;
+  k_mix_digits<FMT == 8><<<dim3(a.cols / 128, 4 * tiles), 64, 0, ctx->stream>>>(d);
+
+  MfmaArgs f;
+  memset(&f, 0, sizeof(f));
+  int nt = 0;
+  for (int m = 0; m < a.nm; m++) {
+    f.m[m].tile0 = nt;
+    nt += (a.m[m].rows + 15) / 16;
+    f.m[m].q = a.m[m].q;
+    f.m[m].s = a.m[m].s;
+    f.m[m].y = a.m[m].y;
+    f.m[m].rows = a.m[m].rows;
+    f.m[m].rb = a.m[m].rb;
+    f.m[m].ng = a.m[m].ng;
+    f.m[m].ldy = a.m[m].ldy;
+  }
+  f.nm = a.nm;
+  f.tiles = nt;
+  f.G = a.cols / 128;
+  f.T = a.B;
+  f.dig = dig;
+  f.asc = d.asc;
+  if (CONV) {
+    f.conv_state = a.conv_state;
+    f.conv_w = a.conv_w;
+    f.mix = a.mix;
+    f.K = a.K;
+    f.conv_slot_stride = a.conv_slot_stride;
+    auto slot = [&](int t) { return a.tok.tab ? a.tok.slot[t] : 0; };
+    auto pos = [&](int t) { return a.tok.tab ? a.tok.pos[t] : a.tok.base + t; };
+    for (int t = 0; t < a.B; t++) {
+      ConvTok &c = f.tok[t];
+      c.slot = slot(t);
+      c.own = (short)(pos(t) % a.K);
+      c.last = 1;
+      for (int u = t + 1; u < a.B; u++)
+        if (slot(u) == slot(t) && pos(u) % a.K == pos(t) % a.K) c.last = 0;
+      for (int k = 0; k < a.K; k++) {
+        // the word as the tokens before this one left it, the token's own
+        // value at its own position
+        const int src = pos(t) - (a.K - 1 - k);
+        c.src[k] = -2;
+        if (src < 0) continue;
+        c.word[k] = (signed char)(src % a.K);
+        c.src[k] = -1;
+        for (int u = 0; u < t; u++)
+          if (slot(u) == slot(t) && pos(u) % a.K == src % a.K) c.src[k] = (signed char)u;
+        if (src == pos(t)) c.src[k] = (signed char)t;
+      }
+    }
+  }
+  const int cus = ctx->sm_count > 0 ? ctx->sm_count : 256;
+  const dim3 grid(nt < cus ? nt : cus, tiles);
+  // several tiles a workgroup: 8 waves that keep the digits; else 16 waves,
+  // twice the loads in flight for the one tile
+  if ((CONV || nt * tiles > cus) && f.G <= 32) {
+    if (f.G <= 16) return launch_mfma<FMT, 8, 2, CONV>(ctx, grid, f);
+    return launch_mfma<FMT, 8, 4, CONV>(ctx, grid, f);
+  }
+  if constexpr (!CONV) {
+    if (f.G <= 16) return launch_mfma<FMT, 16, 1, CONV>(ctx, grid, f);
+    if (f.G <= 32) return launch_mfma<FMT, 16, 2, CONV>(ctx, grid, f);
+  }
+  return launch_mfma<FMT, 16, 4, CONV>(ctx, grid, f);
+}
+
+// The projections of a.B tokens (any number without a convolution).
+template <int FMT, bool CONV>
+int launch_proj(ColiCuda *ctx, const ProjArgs &a, unsigned char *dig) {
+  if (a.B >= kMfmaMinTok && mfma_takes<FMT, CONV>(a)) return launch_proj_mfma<FMT, CONV>(ctx, a, dig);
+  ProjArgs p = a;
+  for (int r0 = 0; r0 < a.B; r0 += kMixMaxTok) {
+    p.B = a.B - r0 < kMixMaxTok ? a.B - r0 : kMixMaxTok;
+    p.x = a.x + (size_t)r0 * a.ldx;
+    for (int m = 0; m < a.nm; m++)
+      if (a.m[m].y) p.m[m].y = a.m[m].y + (size_t)r0 * a.m[m].ldy;
+    launch_proj_vector<FMT, CONV>(ctx, p);
+  }
+  return 0;
 }
 
 ProjMat pmat(const unsigned char *q, const float *s, float *y, int rows, int rb, int ng, int ldy) {
@@ -1138,7 +1265,8 @@ int gdn_run(ColiCuda *ctx, const GdnCall &c) {
                om = ob + align_up((size_t)B * c.vh * 4), oz = om + align_up((size_t)B * C * 4),
                oc = oz + align_up((size_t)B * vd * 4), oy = oc + align_up((size_t)B * vd * 4),
                oms = oy + align_up((size_t)B * H * 4),
-               total = oms + align_up((size_t)B * c.vh * ((c.dv + 31) / 32) * 4);
+               od = oms + align_up((size_t)B * c.vh * ((c.dv + 31) / 32) * 4),
+               total = od + align_up(mix_digit_bytes(B, H > vd ? H : vd));
   if (ensure_scratch(ctx, kScrMixer, total, c.name)) return -1;
   char *w = (char *)ctx->scratch[kScrMixer];
   const float *x = c.x, *av = c.a, *bv = c.b;
@@ -1155,6 +1283,7 @@ int gdn_run(ColiCuda *ctx, const GdnCall &c) {
   }
   float *mix = (float *)(w + om), *z = (float *)(w + oz), *core = (float *)(w + oc), *msp = (float *)(w + oms);
   float *y = c.device_io ? c.out : (float *)(w + oy);
+  unsigned char *dig = (unsigned char *)(w + od);
 
   ProjArgs p;
   memset(&p, 0, sizeof(p));
@@ -1173,7 +1302,7 @@ int gdn_run(ColiCuda *ctx, const GdnCall &c) {
   p.K = c.K;
   p.conv_slot_stride = (long long)c.K * C;
   p.tok = c.tok;
-  launch_proj<4, true>(ctx, p);
+  if (launch_proj<4, true>(ctx, p, dig)) return -1;
 
   GdnArgs g;
   memset(&g, 0, sizeof(g));
@@ -1231,7 +1360,7 @@ int gdn_run(ColiCuda *ctx, const GdnCall &c) {
   o.nsp = nsp;
   o.hw = c.dv;
   o.eps = c.eps;
-  launch_proj<4, false>(ctx, o);
+  if (launch_proj<4, false>(ctx, o, dig)) return -1;
   if (launch_status(c.name)) return -1;
   if (c.device_io) return 0;
   hipError_t e = hipMemcpyAsync(c.out, y, (size_t)B * H * 4, hipMemcpyDeviceToHost, ctx->stream);
@@ -1293,7 +1422,8 @@ int gqa_run(ColiCuda *ctx, const GqaCall &c) {
                ov = ok + align_up((size_t)R * kvrows * 4), oq = ov + align_up((size_t)R * kvrows * 4),
                og = oq + align_up((size_t)R * ctxn * 4), oc = og + align_up((size_t)R * ctxn * 4),
                oy = oc + align_up((size_t)R * ctxn * 4), op = oy + align_up((size_t)R * H * 4),
-               total = op + align_up((size_t)R * c.nkv * S * psz * 4);
+               od = op + align_up((size_t)R * c.nkv * S * psz * 4),
+               total = od + align_up(mix_digit_bytes(R, H > ctxn ? H : ctxn));
   if (ensure_scratch(ctx, kScrMixer, total, c.name)) return -1;
   char *w = (char *)ctx->scratch[kScrMixer];
   const float *x = c.x;
@@ -1305,23 +1435,21 @@ int gqa_run(ColiCuda *ctx, const GqaCall &c) {
   float *qp = (float *)(w + oqp), *kr = (float *)(w + ok), *vr = (float *)(w + ov);
   float *q = (float *)(w + oq), *gate = (float *)(w + og), *cx = (float *)(w + oc);
   float *y = c.device_io ? c.out : (float *)(w + oy), *part = (float *)(w + op);
+  unsigned char *dig = (unsigned char *)(w + od);
 
-  for (int r0 = 0; r0 < R; r0 += kMixMaxTok) {
-    const int n = R - r0 < kMixMaxTok ? R - r0 : kMixMaxTok;
-    ProjArgs p;
-    memset(&p, 0, sizeof(p));
-    p.m[0] = pmat(c.q_q, c.q_s, qp + (size_t)r0 * qrows, qrows, c.q_rb, c.q_ng, qrows);
-    p.m[1] = pmat(c.k_q, c.k_s, kr + (size_t)r0 * kvrows, kvrows, c.k_rb, c.k_ng, kvrows);
-    p.m[2] = pmat(c.v_q, c.v_s, vr + (size_t)r0 * kvrows, kvrows, c.v_rb, c.v_ng, kvrows);
-    p.nm = 3;
-    p.rows_total = qrows + 2 * kvrows;
-    p.x = x + (size_t)r0 * H;
-    p.ldx = H;
-    p.cols = H;
-    p.gs = c.gs;
-    p.B = n;
-    launch_proj<4, false>(ctx, p);
-  }
+  ProjArgs p;
+  memset(&p, 0, sizeof(p));
+  p.m[0] = pmat(c.q_q, c.q_s, qp, qrows, c.q_rb, c.q_ng, qrows);
+  p.m[1] = pmat(c.k_q, c.k_s, kr, kvrows, c.k_rb, c.k_ng, kvrows);
+  p.m[2] = pmat(c.v_q, c.v_s, vr, kvrows, c.v_rb, c.v_ng, kvrows);
+  p.nm = 3;
+  p.rows_total = qrows + 2 * kvrows;
+  p.x = x;
+  p.ldx = H;
+  p.cols = H;
+  p.gs = c.gs;
+  p.B = R;
+  if (launch_proj<4, false>(ctx, p, dig)) return -1;
   PrepArgs pr;
   memset(&pr, 0, sizeof(pr));
   pr.qp = qp;
@@ -1371,23 +1499,17 @@ int gqa_run(ColiCuda *ctx, const GqaCall &c) {
   cb.S = S;
   k_gqa_combine<<<dim3(c.nh * (hd / 64), R), 256, 0, ctx->stream>>>(cb);
 
-  for (int r0 = 0; r0 < R; r0 += kMixMaxTok) {
-    const int n = R - r0 < kMixMaxTok ? R - r0 : kMixMaxTok;
-    ProjArgs o;
-    memset(&o, 0, sizeof(o));
-    o.m[0] = pmat((const unsigned char *)c.o_q, c.o_s, y + (size_t)r0 * H, H, c.o_rb, c.o_ng, H);
-    o.nm = 1;
-    o.rows_total = H;
-    o.x = cx + (size_t)r0 * ctxn;
-    o.ldx = ctxn;
-    o.cols = ctxn;
-    o.gs = c.gs;
-    o.B = n;
-    if (c.o_fmt == 4)
-      launch_proj<4, false>(ctx, o);
-    else
-      launch_proj<8, false>(ctx, o);
-  }
+  ProjArgs o;
+  memset(&o, 0, sizeof(o));
+  o.m[0] = pmat((const unsigned char *)c.o_q, c.o_s, y, H, c.o_rb, c.o_ng, H);
+  o.nm = 1;
+  o.rows_total = H;
+  o.x = cx;
+  o.ldx = ctxn;
+  o.cols = ctxn;
+  o.gs = c.gs;
+  o.B = R;
+  if (c.o_fmt == 4 ? launch_proj<4, false>(ctx, o, dig) : launch_proj<8, false>(ctx, o, dig)) return -1;
   if (launch_status(c.name)) return -1;
   if (c.device_io) return 0;
   hipError_t e = hipMemcpyAsync(c.out, y, (size_t)R * H * 4, hipMemcpyDeviceToHost, ctx->stream);

@@ -1,0 +1,364 @@
+// Mixer projections on the int8 matrix cores, for calls of several tokens.
+//
+//   y[t][row] = sum_g s[row][g] * sum_{i in g} code(row, i) * x[t][i]
+//
+// over int4 rows in groups of 128 or int8 rows with one scale, fp32
+// activations.  Each 128-column group of a token's activations is held as a
+// 30-bit fixed-point number: q = rint(x * 2^k) with 2^k the power of two that
+// brings the group's largest magnitude into [2^29, 2^30), so every value
+// within 2^-6 of that largest one is exact and the others are off by at most
+// 2^-31 of it (less than one fp32 rounding of the group's sum).  q is cut
+// into four balanced base-256 digits, each an MFMA B operand; the four int32
+// dots with the (small, exact) weight codes are exact, and are put together
+// as ((c1 * 256 + c2) * 2^16 + (c3 * 256 + c4)) * 2^-k in fp32: one rounding
+// for the group, then one FMA with the row's group scale.
+//
+// k_mix_digits forms the digits once per call in the MFMA's own lane order;
+// k_mix_mfma streams the weights.
+#pragma once
+
+#include "sw_device.h"
+#include "sw_lds_dma.h"
+
+namespace sw {
+
+constexpr int kDigPlanes = 8;  // four digits x two 64-column halves of a group
+constexpr int kDigTile = 16;   // tokens of one MFMA B operand
+
+// Bytes of the digits and the group scales of `tokens` rows of `cols`.
+inline size_t mix_digit_bytes(int tokens, int cols) {
+  return (size_t)((tokens + kDigTile - 1) / kDigTile) * (cols / 128) * (kDigPlanes * 1024 + kDigTile * 4);
+}
+// The group scales lie behind the digits: [tile][group][16 tokens].
+__host__ __device__ inline size_t mix_digit_scales_at(int tokens, int cols) {
+  return (size_t)((tokens + kDigTile - 1) / kDigTile) * (cols / 128) * (kDigPlanes * 1024);
+}
+
+struct DigitArgs {
+  const float *x;  // token t at x + t * ldx
+  int ldx, cols, T;
+  unsigned char *dig;
+  float *asc;
+  // optional per-(token, head) factor 1/sqrt(sum(msp) / hw + eps)
+  const float *msp;
+  int nsp, hw;
+  float eps;
+};
+
+// Sixteen lanes take one (token, group), eight columns each; a wave takes
+// four tokens of one group.  Digit planes, per (16-token tile, group):
+// [digit d][half h][lane kb * 16 + token][16 bytes].  ROWS8 0 (int4 rows):
+// byte j of half h is column 32 kb + 2 j + h, the low (0) or high (1) nibble
+// of byte j of the 16 that a lane loads; 1 (int8 rows): column
+// 32 kb + 16 h + j.  A group with an infinity or NaN gets the scale NaN.
+// Latency-bound: 4.5 us up to 16 tokens.
+// grid (cols / 128, 4 * tiles), 64 threads.
+template <int ROWS8>
+__global__ __launch_bounds__(64) void k_mix_digits(DigitArgs a) {
+  const int lane = threadIdx.x, i = lane & 15, kb = i >> 2;
+  const int g = blockIdx.x, tile = blockIdx.y >> 2, n = (blockIdx.y & 3) * 4 + (lane >> 4);
+  const int G = a.cols >> 7, t = tile * kDigTile + n, tc = t < a.T ? t : a.T - 1;
+  const int col = g * 128 + 8 * i;
+  const float4 v0 = *(const float4 *)(a.x + (size_t)tc * a.ldx + col);
+  const float4 v1 = *(const float4 *)(a.x + (size_t)tc * a.ldx + col + 4);
+  float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+  if (a.msp) {
+    const float *m = a.msp + ((size_t)tc * (a.cols / a.hw) + col / a.hw) * a.nsp;
+    float ms = 0.0f;
+    for (int k = 0; k < a.nsp; k++) ms += m[k];
+    const float r = 1.f / sqrtf(ms / (float)a.hw + a.eps);
+#pragma unroll
+    for (int e = 0; e < 8; e++) v[e] *= r;
+  }
+  // magnitudes as integers: a NaN orders above infinity
+  unsigned mb = 0;
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    const unsigned b = __float_as_uint(v[e]) & 0x7fffffffu;
+    mb = b > mb ? b : mb;
+  }
+#pragma unroll
+  for (int o = 1; o < 16; o <<= 1) {
+    const unsigned b = (unsigned)__shfl_xor((int)mb, o);
+    mb = b > mb ? b : mb;
+  }
+  const bool bad = mb >= 0x7f800000u;
+  const int k0 = 29 + 127 - (int)(mb >> 23), k = k0 < 120 ? k0 : 120;
+  unsigned d[4][2] = {};
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    int q = bad ? 0 : (int)__builtin_rintf(__builtin_ldexpf(v[e], k));
+    const int w = ROWS8 ? e >> 2 : e & 1, sh = 8 * (ROWS8 ? e & 3 : e >> 1);
+#pragma unroll
+    for (int p = 3; p > 0; p--) {
+      const int lo = (int)(signed char)(q & 255);
+      d[p][w] |= (unsigned)(lo & 255) << sh;
+      q = (q - lo) >> 8;
+    }
+    d[0][w] |= (unsigned)(q & 255) << sh;
+  }
+  unsigned *const out = (unsigned *)a.dig + ((size_t)tile * G + g) * (kDigPlanes * 256) + (kb * 16 + n) * 4;
+#pragma unroll
+  for (int p = 0; p < 4; p++)
+#pragma unroll
+    for (int w = 0; w < 2; w++) {
+      const int half = ROWS8 ? (i & 3) >> 1 : w, dw = ROWS8 ? 2 * (i & 1) + w : i & 3;
+      out[(2 * p + half) * 256 + dw] = d[p][w];
+    }
+  // int4 codes enter the MFMA as 16 * (nibble - 8)
+  if (i == 0)
+    a.asc[((size_t)tile * G + g) * kDigTile + n] =
+        bad ? __builtin_nanf("") : mb == 0 ? 0.0f : __builtin_ldexpf(ROWS8 ? 1.0f : 0.0625f, -k);
+}
+
+// What one token of a Gated DeltaNet call reads and writes in the causal
+// convolution's ring (K <= 4): where each tap's raw value comes from, and
+// whether the token's own raw value is the last one written to its ring word.
+struct ConvTok {
+  signed char src[4];  // -2: before the sequence, -1: the ring in memory, else a token of this call
+  signed char word[4];  // ring word of each tap
+  int slot;
+  short own;   // ring word the token writes
+  short last;  // 1: no later token of the call writes that word
+};
+
+struct MfmaProj {
+  const unsigned char *q;
+  const float *s;
+  float *y;  // y[t * ldy + row]
+  int rows, rb, ng, ldy;
+  int tile0;  // first 16-row tile of the matrix
+};
+
+struct MfmaArgs {
+  MfmaProj m[3];
+  int nm;
+  int tiles;  // 16-row tiles of all matrices
+  int G, T;   // 128-column groups; tokens
+  const unsigned char *dig;
+  const float *asc;
+  // causal convolution on matrix 0
+  float *conv_state;    // [slot][K][channels]
+  const float *conv_w;  // [channels][K]
+  float *mix;           // [T][channels]
+  int K;
+  long long conv_slot_stride;
+  ConvTok tok[kDigTile];
+};
+
+// A persistent workgroup of W waves walks 16-row tiles, b, b + grid, ...;
+// wave w owns GW consecutive 128-column groups of every tile (whole 128-byte
+// lines of a row).  The wave copies its share of the next NR - 1 tiles
+// (weights, group scales, and for the convolution the ring words and tap
+// weights that its own lanes will need) into its slots of an LDS ring
+// (global_load_lds), so the bytes in flight hold no registers and the loop
+// body exists once: launches of a few tiles a workgroup would otherwise spend
+// their time fetching unrolled code.  With 8 waves the tokens' digits stay in
+// registers for the whole launch and come from L2 once per workgroup (8 KB a
+// group against 1 KB of int4 weights a tile); with 16 waves, for launches of
+// one tile a workgroup, they are read for each tile, two groups at a time.
+// Per group: two unpacked A operands (the nibbles, offset by XOR and kept in
+// the high half of their byte), eight MFMAs, one fp32 step.  The waves' sums
+// meet in LDS in wave order, one barrier a tile that leaves the copies in
+// flight; waves 0..3 finish an even tile, 4..7 an odd one, a thread per
+// (row, token).
+// HBM-bound on the weights up to 16 tokens.  Measured at 16 tokens, S397: qkv
+// and z (44.6 MB) 216 -> 17.7 us, out (17.8 MB) 117 -> 12.6 us against the fp32
+// FMA kernel; at one group of registers in flight instead of the ring 25 to
+// 30 and 14 us, with the loop unrolled over register buffers 21 and 17 us.
+// grid (min(tiles, compute units), token tiles), 64 W threads.
+constexpr int kMfmaMaxGroups = 64;  // 128-column groups of a row (W 16, GW 4)
+constexpr int kMfmaPitch = 20;      // floats per token in LDS (16 rows, padded)
+constexpr int kConvCopies = 4;      // dword copies of a tile's convolution: tap weights, three ring words
+
+template <int FMT, int W, int GW, bool CONV>
+struct MfmaRing {
+  static constexpr int NA = FMT == 4 ? 1 : 2;
+  static constexpr int scales = FMT == 4 ? (GW * 16 + 63) / 64 : 1;  // dword copies of a wave's scales
+  static constexpr int wave = GW * NA * 1024 + scales * 256 + (CONV ? kConvCopies * 256 : 0);
+  static constexpr int slot = wave * W;
+  static constexpr int parities = slot > 100 * 1024 ? 1 : 2;  // buffers of the waves' sums
+  static constexpr int red = parities * W * kDigTile * kMfmaPitch * 4;
+  static constexpr int fit = (158 * 1024 - red - 256) / slot;
+  static constexpr int slots = fit < 4 ? fit : 4;
+  static constexpr int lds = slots * slot + red + 256;
+};
+
+template <int FMT, int W, int GW, bool CONV>
+__global__ __launch_bounds__(64 * W) void k_mix_mfma(MfmaArgs a) {
+  typedef MfmaRing<FMT, W, GW, CONV> Ring;
+  constexpr int NA = Ring::NA, NR = Ring::slots, NS = Ring::scales;
+  constexpr int kMfmaRed = Ring::red;
+  constexpr int ND = W == 8 || GW < 2 ? GW : 2;  // digit buffers
+  constexpr bool RES = ND == GW;                 // digits resident
+  constexpr int OPS = GW * NA + NS;              // copies of a tile, at least
+  static_assert(NR >= 1, "a tile fits the LDS");
+  extern __shared__ __align__(16) unsigned char smem[];
+  float *const red = (float *)smem;  // [parity][wave][token][pitch]
+  uint64_t *const etab = (uint64_t *)(smem + kMfmaRed);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, kb = lane >> 4;
+  unsigned char *const ring = smem + kMfmaRed + 256 + wave * (NR * Ring::wave);
+  const int t0 = blockIdx.y * kDigTile, nt = a.T - t0 < kDigTile ? a.T - t0 : kDigTile;
+  const int g0 = wave * GW, tiles = a.tiles, step = gridDim.x;
+  if (CONV && tid < 32) etab[tid] = kExp2Tab[tid];
+  // the token and row that this thread finishes; waves 0..3 even tiles of the
+  // workgroup, 4..7 odd ones
+  const int ft = (tid & 255) >> 4, fr = tid & 15, fpar = wave >> 2;  // waves 8.. finish none
+  ConvTok ct;
+  if (CONV) ct = a.tok[ft < nt ? ft : 0];
+
+  auto mat_of = [&](int t) {
+    int m = 0;
+    if (a.nm > 1 && t >= a.m[1].tile0) m = 1;
+    if (a.nm > 2 && t >= a.m[2].tile0) m = 2;
+    return m;
+  };
+  // lanes of groups past the row read its last group: inside the row, unused
+  auto copy = [&](int t, int i) {
+    const int m = mat_of(t);
+    const MfmaProj &pm = a.m[m];
+    const int row0 = (t - pm.tile0) * 16, row = row0 + n < pm.rows ? row0 + n : pm.rows - 1;
+    unsigned char *const slot = ring + (i % NR) * Ring::wave;
+    const unsigned char *q = pm.q + (size_t)row * pm.rb + (FMT == 4 ? 16 : 32) * kb;
+#pragma unroll
+    for (int j = 0; j < GW; j++) {
+      const int g = g0 + j < a.G ? g0 + j : a.G - 1;
+#pragma unroll
+      for (int h = 0; h < NA; h++)
+        dma_b128(q + (size_t)g * (FMT == 4 ? 64 : 128) + 16 * h, lds_addr(slot + (j * NA + h) * 1024));
+    }
+#pragma unroll
+    for (int j = 0; j < NS; j++) {
+      const int gs = g0 + 4 * j + kb, g = gs < a.G && 4 * j + kb < GW ? gs : a.G - 1;
+      dma_b32(FMT == 4 ? pm.s + (size_t)row * pm.ng + g : pm.s + row, lds_addr(slot + GW * NA * 1024 + j * 256));
+    }
+    if (CONV && m == 0 && (i & 1) == fpar) {
+      const int ch = row0 + fr < pm.rows ? row0 + fr : pm.rows - 1, k = lane >> 4;
+      unsigned char *const cw = slot + GW * NA * 1024 + NS * 256;
+      dma_b32(a.conv_w + (size_t)ch * a.K + (k < a.K ? k : 0), lds_addr(cw));
+      const float *cs = a.conv_state + (size_t)ct.slot * a.conv_slot_stride + ch;
+#pragma unroll
+      for (int j = 0; j < 3; j++) dma_b32(cs + (size_t)ct.word[j] * pm.rows, lds_addr(cw + (j + 1) * 256));
+    }
+  };
+
+  copy(blockIdx.x, 0);
+  // lanes of absent tokens read token 0's digits: no more lines
+  const unsigned char *const dp =
+      a.dig + (size_t)blockIdx.y * a.G * (kDigPlanes * 1024) + (kb * 16 + (n < nt ? n : 0)) * 16;
+  const float *const ap = a.asc + (size_t)blockIdx.y * a.G * kDigTile + (n < nt ? n : 0);
+  v4i dv[ND][kDigPlanes];
+  float av[GW];
+  auto digits = [&](int b, int g) {
+    const int gc = g < a.G ? g : a.G - 1;
+#pragma unroll
+    for (int d = 0; d < kDigPlanes; d++) dv[b][d] = *(const v4i *)(dp + ((size_t)gc * kDigPlanes + d) * 1024);
+  };
+#pragma unroll
+  for (int i = 0; i < GW; i++) av[i] = g0 + i < a.G ? ap[(size_t)(g0 + i) * kDigTile] : 0.0f;
+  if (RES) {
+#pragma unroll
+    for (int i = 0; i < ND; i++) digits(i, g0 + i);
+#pragma unroll
+    for (int i = 0; i < ND; i++)
+#pragma unroll
+      for (int d = 0; d < kDigPlanes; d++) asm volatile("" : "+v"(dv[i][d]));
+  }
+#pragma unroll
+  for (int i = 0; i < GW; i++) asm volatile("" : "+v"(av[i]));
+  for (int i = 1; i < NR - 1; i++)
+    if ((int)blockIdx.x + i * step < tiles) copy(blockIdx.x + i * step, i);
+
+  for (int t = blockIdx.x, i = 0; t < tiles; t += step, i++) {
+    const int m = mat_of(t), p = i & 1;
+    const MfmaProj &pm = a.m[m];
+    // the slot the next copy fills was read a tile ago
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    const bool more = t + (NR - 1) * step < tiles;
+    if (NR > 1 ? more : i > 0) copy(t + (NR - 1) * step, i + NR - 1);
+    // this tile's copies are done when no more than the younger tiles' are left
+    if (NR > 1 && more) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NR - 1) * OPS) : "memory");
+    } else {
+      wait_dma();
+    }
+    const unsigned char *const slot = ring + (i % NR) * Ring::wave;
+    const float *const sc = (const float *)(slot + GW * NA * 1024);
+    v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
+    auto group = [&](int j, int b, float as) {
+      v4i a0, a1;
+      if (FMT == 4) {
+        const v4u w = *(const v4u *)(slot + j * 1024 + 16 * lane);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const unsigned x = w[e] ^ 0x88888888u;
+          a0[e] = (int)((x << 4) & 0xF0F0F0F0u);
+          a1[e] = (int)(x & 0xF0F0F0F0u);
+        }
+      } else {
+        a0 = *(const v4i *)(slot + (2 * j) * 1024 + 16 * lane);
+        a1 = *(const v4i *)(slot + (2 * j + 1) * 1024 + 16 * lane);
+      }
+      v4i c[4];
+#pragma unroll
+      for (int d = 0; d < 4; d++) c[d] = mfma_i8(a0, dv[b][2 * d], v4i{0, 0, 0, 0});
+#pragma unroll
+      for (int d = 0; d < 4; d++) c[d] = mfma_i8(a1, dv[b][2 * d + 1], c[d]);
+      v4f s4 = v4f{1.f, 1.f, 1.f, 1.f};
+      if (FMT == 4) s4 = *(const v4f *)(sc + 16 * j + 4 * kb);
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const float f = __builtin_fmaf((float)(c[0][e] * 256 + c[1][e]), 65536.0f, (float)(c[2][e] * 256 + c[3][e]));
+        acc[e] = __builtin_fmaf(f, s4[e] * as, acc[e]);
+      }
+    };
+    // groups past the row add their scale 0
+    if (RES) {
+#pragma unroll
+      for (int j = 0; j < GW; j++) group(j, j % ND, av[j]);
+    } else {
+      digits(0, g0);
+#pragma unroll
+      for (int j = 0; j < GW; j += 2) {
+        digits(1, g0 + j + 1);
+        group(j, 0, av[j]);
+        if (j + 2 < GW) digits(0, g0 + j + 2);
+        group(j + 1, 1, av[j + 1]);
+      }
+    }
+    *(v4f *)(red + ((p % Ring::parities * W + wave) * kDigTile + n) * kMfmaPitch + 4 * kb) = acc;
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    const int row = (t - pm.tile0) * 16 + fr;
+    if (p == fpar && ft < nt && row < pm.rows) {
+      auto raw = [&](int tok) {
+        const float *r = red + (p % Ring::parities * W * kDigTile + tok) * kMfmaPitch + fr;
+        float v = r[0];
+#pragma unroll
+        for (int w = 1; w < W; w++) v += r[w * kDigTile * kMfmaPitch];
+        return v;
+      };
+      const float own = raw(ft);
+      if (!CONV || m != 0) {
+        pm.y[(size_t)(t0 + ft) * pm.ldy + row] = FMT == 8 ? own * sc[fr] : own;
+      } else {
+        // the taps in order (c/qwen.c:3018-3023)
+        const float *cw = (const float *)(slot + GW * NA * 1024 + NS * 256);
+        float sconv = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          const int src = ct.src[k];
+          if (k >= a.K || src == -2) continue;
+          const float v = src == ft ? own : src >= 0 ? raw(src) : cw[64 * (k < 3 ? k + 1 : 0) + lane];
+          sconv = __builtin_fmaf(cw[16 * k + fr], v, sconv);
+        }
+        a.mix[(size_t)ft * pm.rows + row] = silu_ref_t(sconv, etab);
+        // tokens of one sequence share ring words: all of the tile's were
+        // copied to LDS before the barrier
+        if (ct.last) a.conv_state[(size_t)ct.slot * a.conv_slot_stride + (size_t)ct.own * pm.rows + row] = own;
+      }
+    }
+    if (Ring::parities == 1) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  }
+}
+
+}  // namespace sw
