@@ -1191,6 +1191,28 @@ int launch_proj_mfma(ColiCuda *ctx, const ProjArgs &a, unsigned char *dig) {
     }
   }
   const int cus = ctx->sm_count > 0 ? ctx->sm_count : 256;
+  if constexpr (!CONV) {
+    // k_mix_gemm takes 2.9 us per round of workgroups and 128-column group,
+    // k_mix_mfma 0.09 us per 16 tokens, group and round of row tiles, or 0.16
+    // where a round is one tile a workgroup (S397 q, k and v: 1,000 tokens 464
+    // against 736 us, 300 tokens 186 against 222, 160 tokens 186 against 117;
+    // o, 1,000 tokens, 180 against 628)
+    int blocks = 0;
+    for (int m = 0; m < a.nm; m++) blocks += (a.m[m].rows + kGemmRows - 1) / kGemmRows;
+    const int tb = (a.B + kGemmTokens - 1) / kGemmTokens;
+    const long long rounds = ((long long)blocks * tb + cus - 1) / cus;
+    if ((nt > cus ? 32 : 16) * rounds * cus < (long long)tiles * nt) {
+      for (int m = 0, at = 0; m < a.nm; m++) {
+        f.m[m].tile0 = at;
+        at += (a.m[m].rows + kGemmRows - 1) / kGemmRows;
+      }
+      const hipError_t e =
+          hipFuncSetAttribute((const void *)k_mix_gemm<FMT>, hipFuncAttributeMaxDynamicSharedMemorySize, kGemmLds);
+      if (e != hipSuccess) return fail_hip("mixer projection attributes", e);
+      k_mix_gemm<FMT><<<blocks * tb, 512, kGemmLds, ctx->stream>>>(f);
+      return 0;
+    }
+  }
   const dim3 grid(nt < cus ? nt : cus, tiles);
   // several tiles a workgroup: 8 waves that keep the digits; else 16 waves,
   // twice the loads in flight for the one tile

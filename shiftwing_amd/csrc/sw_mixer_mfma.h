@@ -361,4 +361,142 @@ __global__ __launch_bounds__(64 * W) void k_mix_mfma(MfmaArgs a) {
   }
 }
 
+// The same product for prompt chunks: a workgroup of 8 waves computes 128 rows
+// x 128 tokens, a wave 64 rows x 32 tokens (two waves along the rows).  Per
+// 128-column group the workgroup's digit planes (64 KB) and scales go to one
+// of two LDS buffers by global_load_lds while the previous group is worked on;
+// a wave's own weight bytes go to registers.  A wave unpacks a row tile once
+// for its two token tiles and reads a token tile's digits once for its four
+// row tiles.  Workgroups of one token block follow each other by the number
+// of token blocks, so that with eight of them an XCD's L2 keeps one block's
+// digits.
+// Bound by MFMA (64 of 16 cycles a wave and group) and the fp32 steps (28 VALU
+// instructions per eight MFMAs) that two waves a SIMD overlap only in part:
+// 2.9 us a group where the MFMAs alone take 0.85.  1,000 tokens, S397: q, k and
+// v 736 -> 464 us, o 628 -> 180 us against k_mix_mfma, 1.3 int8 POP/s.
+// grid row blocks x token blocks, 512 threads.
+constexpr int kGemmRows = 128, kGemmTokens = 128;
+constexpr int kGemmTiles = kGemmTokens / kDigTile;
+constexpr int kGemmScales = kGemmTiles * kDigPlanes * 1024;  // activation, then row scales
+constexpr int kGemmBuf = kGemmScales + kGemmTokens * 4 + kGemmRows * 4;
+constexpr int kGemmLds = 2 * kGemmBuf;
+
+template <int FMT>
+__global__ __launch_bounds__(512) void k_mix_gemm(MfmaArgs a) {
+  constexpr int NA = FMT == 4 ? 1 : 2, RT = 4, NTW = 2;
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, kb = lane >> 4;
+  const int wm = wave & 1, wn = wave >> 1;
+  const int ttiles = (a.T + kDigTile - 1) / kDigTile, tb = (ttiles + kGemmTiles - 1) / kGemmTiles;
+  const int rb = blockIdx.x / tb, tile0 = (blockIdx.x % tb) * kGemmTiles;
+  int mi = 0;
+  if (a.nm > 1 && rb >= a.m[1].tile0) mi = 1;
+  if (a.nm > 2 && rb >= a.m[2].tile0) mi = 2;
+  const MfmaProj &pm = a.m[mi];
+  const int row0 = (rb - pm.tile0) * kGemmRows, rlast = pm.rows - 1;
+  const unsigned char *qp[RT];
+#pragma unroll
+  for (int r = 0; r < RT; r++) {
+    const int row = row0 + 64 * wm + 16 * r + n;
+    qp[r] = pm.q + (size_t)(row < rlast ? row : rlast) * pm.rb + (FMT == 4 ? 16 : 32) * kb;
+  }
+  v4u w[RT][NA], wn1[RT][NA];
+  auto weights = [&](int g) {
+#pragma unroll
+    for (int r = 0; r < RT; r++)
+#pragma unroll
+      for (int h = 0; h < NA; h++) wn1[r][h] = *(const v4u *)(qp[r] + (size_t)g * (FMT == 4 ? 64 : 128) + 16 * h);
+  };
+  // one group's digits and scales; token tiles past the last repeat it
+  auto copy = [&](int g, int b) {
+    unsigned char *const buf = smem + b * kGemmBuf;
+#pragma unroll
+    for (int j = 0; j < kGemmTiles; j++) {  // wave w copies plane w of every tile
+      const int tt = tile0 + j < ttiles ? tile0 + j : ttiles - 1;
+      dma_b128(a.dig + (((size_t)tt * a.G + g) * kDigPlanes + wave) * 1024 + 16 * lane,
+               lds_addr(buf + (j * kDigPlanes + wave) * 1024));
+    }
+    if (wave < NTW) {
+      const int j = 4 * wave + kb, tt = tile0 + j < ttiles ? tile0 + j : ttiles - 1;
+      dma_b32(a.asc + ((size_t)tt * a.G + g) * kDigTile + n, lds_addr(buf + kGemmScales + wave * 256));
+    }
+    if (FMT == 4 && wave >= 6) {
+      const int row = row0 + 64 * (wave - 6) + lane;
+      dma_b32(pm.s + (size_t)(row < rlast ? row : rlast) * pm.ng + g,
+              lds_addr(buf + kGemmScales + kGemmTokens * 4 + (wave - 6) * 256));
+    }
+  };
+  v4f acc[RT][NTW];
+#pragma unroll
+  for (int r = 0; r < RT; r++)
+#pragma unroll
+    for (int j = 0; j < NTW; j++) acc[r][j] = v4f{0.f, 0.f, 0.f, 0.f};
+  copy(0, 0);
+  weights(0);
+  for (int g = 0; g < a.G; g++) {
+    const unsigned char *const buf = smem + (g & 1) * kGemmBuf;
+    // this group's copies have landed and every wave has left the other buffer
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+    for (int r = 0; r < RT; r++)
+#pragma unroll
+      for (int h = 0; h < NA; h++) w[r][h] = wn1[r][h];
+    if (g + 1 < a.G) {
+      copy(g + 1, (g + 1) & 1);
+      weights(g + 1);
+    }
+    v4i aop[RT][2];
+    v4f s4[RT];
+#pragma unroll
+    for (int r = 0; r < RT; r++) {
+      if (FMT == 4) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const unsigned x = w[r][0][e] ^ 0x88888888u;
+          aop[r][0][e] = (int)((x << 4) & 0xF0F0F0F0u);
+          aop[r][1][e] = (int)(x & 0xF0F0F0F0u);
+        }
+        s4[r] = *(const v4f *)(buf + kGemmScales + kGemmTokens * 4 + (64 * wm + 16 * r + 4 * kb) * 4);
+      } else {
+        aop[r][0] = __builtin_bit_cast(v4i, w[r][0]);
+        aop[r][1] = __builtin_bit_cast(v4i, w[r][NA - 1]);
+        s4[r] = v4f{1.f, 1.f, 1.f, 1.f};
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NTW; j++) {
+      const int tl = wn * NTW + j;
+      v4i d[kDigPlanes];
+#pragma unroll
+      for (int p = 0; p < kDigPlanes; p++) d[p] = *(const v4i *)(buf + (tl * kDigPlanes + p) * 1024 + 16 * lane);
+      const float as = *(const float *)(buf + kGemmScales + (tl * kDigTile + n) * 4);
+#pragma unroll
+      for (int r = 0; r < RT; r++) {
+        v4i c[4];
+#pragma unroll
+        for (int p = 0; p < 4; p++) c[p] = mfma_i8(aop[r][0], d[2 * p], v4i{0, 0, 0, 0});
+#pragma unroll
+        for (int p = 0; p < 4; p++) c[p] = mfma_i8(aop[r][1], d[2 * p + 1], c[p]);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const float f = __builtin_fmaf((float)(c[0][e] * 256 + c[1][e]), 65536.0f, (float)(c[2][e] * 256 + c[3][e]));
+          acc[r][j][e] = __builtin_fmaf(f, s4[r][e] * as, acc[r][j][e]);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < NTW; j++) {
+    const int t = (tile0 + wn * NTW + j) * kDigTile + n;
+    if (t >= a.T) continue;
+#pragma unroll
+    for (int r = 0; r < RT; r++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int row = row0 + 64 * wm + 16 * r + 4 * kb + e;
+        if (row <= rlast) pm.y[(size_t)t * pm.ldy + row] = FMT == 8 ? acc[r][j][e] * pm.s[row] : acc[r][j][e];
+      }
+  }
+}
+
 }  // namespace sw

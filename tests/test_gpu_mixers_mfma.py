@@ -51,7 +51,9 @@ def test_gdn_projection_edges(be, oracle, H, kh, vh, dk, dv, K, slots, pos):
 
 
 @pytest.mark.parametrize("H,nh,nkv,o_fmt,rows", [(128, 2, 2, 4, 2), (128, 2, 1, 1, 15), (256, 4, 2, 4, 17),
-                                                 (2304, 32, 2, 1, 33), (2304, 66, 6, 4, 16)])
+                                                 (2304, 32, 2, 1, 33), (2304, 66, 6, 4, 16),
+                                                 # enough row and token tiles for the 128 x 128 blocks, both ragged
+                                                 (256, 160, 10, 4, 401), (128, 144, 9, 1, 1025)])
 def test_gqa_projection_edges(be, oracle, H, nh, nkv, o_fmt, rows):
     from oracle import pyoracle as po
     at = po.HostAttn(61, H, nh, nkv, 64, 32, o_fmt=o_fmt)
@@ -60,8 +62,14 @@ def test_gqa_projection_edges(be, oracle, H, nh, nkv, o_fmt, rows):
     rng = np.random.default_rng(62)
     X = _x(rng, rows, H)
     print(f"[gqa edges] H={H} heads {nh} rows {rows} o_fmt {o_fmt}", flush=True)
-    want = np.stack([po.oracle_attn_step(oracle, at, X[r], r, kc, vc) for r in range(rows)])
     got = dev.prefill(X, 0)
+    # every token of a small call; from 64 on the first, the last and some between
+    some = range(rows) if rows <= 64 else [0, 15, 16, 127, 128, rows - 2, rows - 1]
+    if rows > 64:  # the keys and values of the others are the device's own, checked at the rows below
+        dk, dv = dev.read_cache()
+        kc[:], vc[:] = dk[0], dv[0]
+    want = np.stack([po.oracle_attn_step(oracle, at, X[r], r, kc, vc) for r in some])
+    got = got[list(some)]
     assert_close_rms(got, want, 1e-4, "output")
     dk, dvv = dev.read_cache()
     assert_close_rms(dk[0][:rows].ravel(), kc[:rows].ravel(), 1e-4, "k cache")
