@@ -31,25 +31,68 @@ using namespace sw;
 // bit: ms = rn(ms + rn(x_i*x_i)) in element order (the serial chain the
 // reference's flags compile), r = 1/sqrtf(ms/n + eps) (correctly rounded
 // division and square root), y_i = rn(rn(x_i*r)*rn(1+w_i)).  One block per
-// row: the block writes a chunk of squares to LDS, one lane adds them in
-// order, the next chunk follows.
+// row: the block writes a chunk of squares to LDS, one wave adds them in
+// order (serial_sum_nonneg), the next chunk follows.
+// Aligned rows of n <= 4096: one read of x as float4, kept in registers with
+// the weights while the sum is formed.  512 rows of 2,048: 18.4 -> 11 us (7.5 us
+// before without its sum).
 constexpr int kNormChunk = 4096;
+__global__ __launch_bounds__(256) static void k_rmsnorm_zero4(float *y, const float *x, const float *w, int n,
+                                                              float eps) {
+  __shared__ __align__(16) float sq[kNormChunk];
+  __shared__ float s_r;
+  constexpr int V = kNormChunk / 4 / 256;
+  const float4 *xs = (const float4 *)(x + (size_t)blockIdx.x * n);
+  float4 xv[V], wv[V];
+  const int np = (n + kSerialStep - 1) / kSerialStep * kSerialStep;
+#pragma unroll
+  for (int k = 0; k < V; k++) {
+    const int i = threadIdx.x + 256 * k;
+    xv[k] = 4 * i < n ? xs[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+#pragma unroll
+  for (int k = 0; k < V; k++) {
+    const int i = threadIdx.x + 256 * k;
+    wv[k] = 4 * i < n ? ((const float4 *)w)[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+#pragma unroll
+  for (int k = 0; k < V; k++) {
+    const int i = threadIdx.x + 256 * k;
+    if (4 * i < np)
+      ((float4 *)sq)[i] = make_float4(__fmul_rn(xv[k].x, xv[k].x), __fmul_rn(xv[k].y, xv[k].y),
+                                      __fmul_rn(xv[k].z, xv[k].z), __fmul_rn(xv[k].w, xv[k].w));
+  }
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    const float ms = serial_sum_nonneg(sq, n, 0.0f);
+    if (threadIdx.x == 0) s_r = 1.0f / sqrtf(ms / (float)n + eps);
+  }
+  __syncthreads();
+  const float r = s_r;
+  float4 *ys = (float4 *)(y + (size_t)blockIdx.x * n);
+#pragma unroll
+  for (int k = 0; k < V; k++) {
+    const int i = threadIdx.x + 256 * k;
+    if (4 * i < n)
+      ys[i] = make_float4(__fmul_rn(__fmul_rn(xv[k].x, r), 1.0f + wv[k].x), __fmul_rn(__fmul_rn(xv[k].y, r), 1.0f + wv[k].y),
+                          __fmul_rn(__fmul_rn(xv[k].z, r), 1.0f + wv[k].z), __fmul_rn(__fmul_rn(xv[k].w, r), 1.0f + wv[k].w));
+  }
+}
+
+// any length and alignment
 __global__ __launch_bounds__(256) static void k_rmsnorm_zero(float *y, const float *x, const float *w, int n,
                                                              float eps) {
-  __shared__ float sq[kNormChunk];
+  __shared__ __align__(16) float sq[kNormChunk];
   __shared__ float s_r;
   const float *xs = x + (size_t)blockIdx.x * n;
   float *ys = y + (size_t)blockIdx.x * n;
   float ms = 0.0f;
   for (int c0 = 0; c0 < n; c0 += kNormChunk) {
     const int m = n - c0 < kNormChunk ? n - c0 : kNormChunk;
-    for (int i = threadIdx.x; i < m; i += blockDim.x) sq[i] = __fmul_rn(xs[c0 + i], xs[c0 + i]);
+    const int mp = (m + kSerialStep - 1) / kSerialStep * kSerialStep;
+    for (int i = threadIdx.x; i < mp; i += blockDim.x) sq[i] = i < m ? __fmul_rn(xs[c0 + i], xs[c0 + i]) : 0.0f;
     __syncthreads();
-    if (threadIdx.x == 0) {
-      const int m64 = m / 64 * 64;
-      ms = serial_sum_lds(sq, m64, ms);
-      for (int i = m64; i < m; i++) ms = __fadd_rn(ms, sq[i]);
-    }
+    if (threadIdx.x < 64) ms = serial_sum_nonneg(sq, m, ms);
     __syncthreads();
   }
   if (threadIdx.x == 0) s_r = 1.0f / sqrtf(ms / (float)n + eps);
@@ -58,10 +101,17 @@ __global__ __launch_bounds__(256) static void k_rmsnorm_zero(float *y, const flo
   for (int i = threadIdx.x; i < n; i += blockDim.x) ys[i] = __fmul_rn(__fmul_rn(xs[i], r), 1.0f + w[i]);
 }
 
+static void launch_rmsnorm(ColiCuda *ctx, float *y, const float *x, const float *w, int batch, int n, float eps) {
+  if (n <= kNormChunk && n % 4 == 0 && (((uintptr_t)x | (uintptr_t)y | (uintptr_t)w) & 15) == 0)
+    k_rmsnorm_zero4<<<batch, 256, 0, ctx->stream>>>(y, x, w, n, eps);
+  else
+    k_rmsnorm_zero<<<batch, 256, 0, ctx->stream>>>(y, x, w, n, eps);
+}
+
 extern "C" int coli_cuda_rmsnorm_zero(ColiCuda *ctx, float *y, const float *x, const float *w, int n,
                                       float eps) {
   if (!ctx || !y || !x || !w || n <= 0) return fail_arg("coli_cuda_rmsnorm_zero: invalid argument");
-  k_rmsnorm_zero<<<1, 256, 0, ctx->stream>>>(y, x, w, n, eps);
+  launch_rmsnorm(ctx, y, x, w, 1, n, eps);
   return launch_status("k_rmsnorm_zero");
 }
 
@@ -69,7 +119,7 @@ extern "C" int coli_cuda_rmsnorm_zero_batch(ColiCuda *ctx, float *y, const float
                                             int batch, int n, float eps) {
   if (!ctx || !y || !x || !w || batch <= 0 || n <= 0)
     return fail_arg("coli_cuda_rmsnorm_zero_batch: invalid argument");
-  k_rmsnorm_zero<<<batch, 256, 0, ctx->stream>>>(y, x, w, n, eps);
+  launch_rmsnorm(ctx, y, x, w, batch, n, eps);
   return launch_status("k_rmsnorm_zero_batch");
 }
 

@@ -9,8 +9,9 @@
 //       IDOT of qmat_mul_ex / qmat_mul_batch for an int8 matrix
 //       (c/qwen.c:1696-1705, 1765-1768, 3313-3319; allow_idot = 1 at 4512-4513
 //       and 4616).
-// The projection streams the vocab x hidden int8 matrix once per group of up
-// to four tokens (HBM-bound: 1.02 GB for 248,320 x 4096).  Each lane keeps
+// The projection streams the vocab x hidden int8 matrix (HBM-bound: 1.02 GB
+// for 248,320 x 4096), once per 16 tokens on the matrix cores (k_head_mfma) and
+// for one to three tokens by VALU dots (k_head_q8): each lane keeps
 // its 16-byte column chunks of the quantised activations in registers; a
 // wave takes kHeadRows rows (one: 1, 2, 4 and 8 measured 5,750, 5,680, 5,520
 // and 5,420 calls/s at S397), loads every chunk of them before the first
@@ -28,21 +29,19 @@ namespace {
 typedef int v4i __attribute__((ext_vector_type(4)));
 
 // rmsnorm_zero then qrow_i8, one token per block.  The sum of squares is the
-// reference's serial chain, run by one thread over products computed in
+// reference's serial chain, run by one wave over products computed in
 // parallel (each product rounds once, as x[i]*x[i] does before the add).
 __global__ __launch_bounds__(256) void k_head_norm(signed char *xq, float *sx, float *hidden, const float *x,
                                                    const float *w, int n, float eps, int pitch) {
-  extern __shared__ float hp[];  // [n]: squares, then the normalised row
+  extern __shared__ float hp[];  // [n, to the next kSerialStep]: squares, then the normalised row
   __shared__ float s_r, red[4];
   const float *xs = x + (size_t)blockIdx.x * n;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) hp[i] = xs[i] * xs[i];
+  const int np = (n + kSerialStep - 1) / kSerialStep * kSerialStep;
+  for (int i = threadIdx.x; i < np; i += blockDim.x) hp[i] = i < n ? xs[i] * xs[i] : 0.0f;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    // LDS reads of the next 32 squares issued before the current 32 adds
-    const int n64 = n / 64 * 64;
-    float ms = serial_sum_lds(hp, n64);
-    for (int i = n64; i < n; i++) ms = __fadd_rn(ms, hp[i]);
-    s_r = 1.0f / sqrtf(ms / (float)n + eps);
+  if (threadIdx.x < 64) {
+    const float ms = serial_sum_nonneg(hp, n, 0.0f);
+    if (threadIdx.x == 0) s_r = 1.0f / sqrtf(ms / (float)n + eps);
   }
   __syncthreads();
   const float r = s_r;
@@ -128,6 +127,69 @@ __global__ __launch_bounds__(256) void k_head_q8(float *logits, const signed cha
   }
 }
 
+// Several tokens: exact int32 dots of 16 rows x up to 16 tokens by
+// v_mfma_i32_16x16x64_i8, so the matrix is streamed once per 16 tokens and the
+// dots leave the VALU (8 tokens, S397: two passes of VALU dots at 268 us each
+// before, one of 203 us now, 5.0 TB/s; eight steps in flight against 4 and 16,
+// nontemporal loads against plain ones: 224 against 232, 223 and 229 us a call).  The quantised activations wait in LDS in the
+// MFMA's lane order ([64-column step][lane][16 bytes], zero past cols and
+// batch); a wave walks 16-row tiles, eight steps (512 contiguous bytes of each
+// row) of weights in flight ahead of the eight it works on, also across
+// tiles.  HBM-bound.  Two workgroups a compute unit fit up to 4,096 columns.
+// grid workgroups of 8 waves, cols % 64 == 0, 16-byte rows.
+constexpr int kHeadSteps = 8;   // steps of 64 columns in flight
+constexpr int kHeadTokens = 16;
+__host__ __device__ inline int head_cols(int cols) { return (cols + 64 * kHeadSteps - 1) / (64 * kHeadSteps) * (64 * kHeadSteps); }
+
+__global__ __launch_bounds__(512) void k_head_mfma(float *logits, const signed char *xq, const float *sx, int pitch,
+                                                   int batch, const signed char *q, const float *scales, int rows,
+                                                   int cols, int row_bytes) {
+  extern __shared__ __align__(16) unsigned char hx[];
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, kb = lane >> 4;
+  const int tiles = (rows + 15) / 16, step = gridDim.x * 8, chunks = head_cols(cols) / (64 * kHeadSteps);
+  int tile = blockIdx.x * 8 + (tid >> 6);
+  v4i cur[kHeadSteps], nxt[kHeadSteps];
+  auto load = [&](int t, int c) {
+    const int row = 16 * t + n < rows ? 16 * t + n : rows - 1;
+    const signed char *p = q + (size_t)row * row_bytes;
+#pragma unroll
+    for (int j = 0; j < kHeadSteps; j++) {
+      const int col = (c * kHeadSteps + j) * 64 + 16 * kb;
+      nxt[j] = __builtin_nontemporal_load((const v4i *)(p + (col < cols ? col : 0)));
+    }
+  };
+  if (tile < tiles) load(tile, 0);
+  for (int u = tid; u < head_cols(cols); u += 512) {
+    const int t = u & 15, col = (u >> 6) * 64 + ((u >> 4) & 3) * 16;
+    ((v4i *)hx)[u] = t < batch && col < cols ? *(const v4i *)(xq + (size_t)t * pitch + col) : v4i{0, 0, 0, 0};
+  }
+  __syncthreads();
+  const float sn = sx[n < batch ? n : 0];
+  for (; tile < tiles; tile += step) {
+    v4i acc = v4i{0, 0, 0, 0};
+    float sc[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) sc[i] = scales[16 * tile + 4 * kb + i < rows ? 16 * tile + 4 * kb + i : rows - 1];
+    for (int c = 0; c < chunks; c++) {
+#pragma unroll
+      for (int j = 0; j < kHeadSteps; j++) cur[j] = nxt[j];
+      if (c + 1 < chunks)
+        load(tile, c + 1);
+      else if (tile + step < tiles)
+        load(tile + step, 0);
+#pragma unroll
+      for (int j = 0; j < kHeadSteps; j++) acc = mfma_i8(cur[j], ((const v4i *)hx)[(c * kHeadSteps + j) * 64 + lane], acc);
+    }
+    if (n < batch) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int row = 16 * tile + 4 * kb + i;
+        if (row < rows) logits[(size_t)n * rows + row] = ((float)acc[i] * sc[i]) * sn;
+      }
+    }
+  }
+}
+
 // any shape: one wave per (row, token), dword dots where aligned
 __global__ __launch_bounds__(256) void k_head_q8_any(float *logits, const signed char *xq, const float *sx,
                                                      int pitch, const signed char *q, const float *scales,
@@ -170,7 +232,7 @@ extern "C" int coli_cuda_output_head_q8(ColiCuda *ctx, float *logits, float *hid
   signed char *xq = (signed char *)ctx->scratch[kScrHead];
   float *sx = (float *)((char *)ctx->scratch[kScrHead] + qbytes);
   hipStream_t st = ctx->stream;
-  const size_t lds = (size_t)cols * sizeof(float);
+  const size_t lds = (size_t)((cols + kSerialStep - 1) / kSerialStep * kSerialStep) * sizeof(float);
   if (lds > 64 * 1024) {
     hipError_t e = hipFuncSetAttribute((const void *)k_head_norm, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return fail_hip("output head norm attributes", e);
@@ -179,6 +241,20 @@ extern "C" int coli_cuda_output_head_q8(ColiCuda *ctx, float *logits, float *hid
   const bool fast = cols % 16 == 0 && row_bytes % 16 == 0 && ((uintptr_t)q & 15) == 0 && cols <= 8192;
   const int nch = (cols + 1023) / 1024;
   const int nchp = nch <= 1 ? 1 : nch <= 2 ? 2 : nch <= 4 ? 4 : 8;
+  // 1 / 2 / 4 / 8 tokens, MFMA against VALU dots: 2,048 columns 105 / 106 / 108 /
+  // 114 against 95 / 115 / 154 / 293 us, 4,096 columns 210 / 211 / 215 / 224 against
+  // 165 / 189 / 278 / 534 (three tokens 113 against 105 at a vocabulary of 100,003)
+  if (fast && batch >= (cols <= 2048 ? 2 : 4) && cols % 64 == 0) {
+    const int hl = head_cols(cols) * 16, cus = ctx->sm_count > 0 ? ctx->sm_count : 256;
+    const hipError_t e = hipFuncSetAttribute((const void *)k_head_mfma, hipFuncAttributeMaxDynamicSharedMemorySize, hl);
+    if (e != hipSuccess) return fail_hip("output head attributes", e);
+    const int wgs = (vocab + 127) / 128, most = cus * (hl <= 72 * 1024 ? 2 : 1);
+    for (int b0 = 0; b0 < batch; b0 += kHeadTokens)
+      k_head_mfma<<<wgs < most ? wgs : most, 512, hl, st>>>(logits + (size_t)b0 * vocab, xq + (size_t)b0 * pitch, sx + b0,
+                                                           pitch, batch - b0 < kHeadTokens ? batch - b0 : kHeadTokens, q,
+                                                           scales, vocab, cols, row_bytes);
+    return launch_status("coli_cuda_output_head_q8");
+  }
   for (int b0 = 0; b0 < batch; b0 += 4) {
     const int nb = batch - b0 < 4 ? batch - b0 : 4;
     float *lg = logits + (size_t)b0 * vocab;

@@ -260,6 +260,101 @@ __device__ __forceinline__ float serial_sum_lds(const float *p, int m, float s =
   return s;
 }
 
+// The same serial chain over terms that are all >= 0 (or NaN), by one whole
+// wave: s = rn(s + p[i]) for i < m in order.  p is LDS, zero beyond m up to the
+// next multiple of kSerialStep; every lane returns the sum.
+// While s = S u stays in one binade [2^23 u, 2^24 u), u its last place,
+// rn(s + p) = (S + rint(p / u)) u, where a p / u halfway between two integers
+// goes to the even sum; so a run of adds is one integer sum.  512 terms a
+// step, eight a lane: the lanes add their rounded terms and scan; the step's
+// first tie is settled from the parity of the sum before it.  The first lane
+// with a second tie, a term of 2^23 u or more, or a sum that reaches 2^24 u
+// ends the run: its terms are added as written and the rest go on from there.
+// A sum that grows from its first terms has one binade step and about one tie
+// per doubling; the first 64 terms, where every few end a run, are added one by
+// one, and so are sums too small or large for exact scaling.  A run is about 750 cycles of dependent code: 2,048 squares in 11 us by
+// one lane's dependent adds, 5 us this way.
+constexpr int kSerialStep = 512;
+__device__ __forceinline__ float lane_value(float v, int l) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
+}
+__device__ __forceinline__ float serial_sum_nonneg(const float *p, int m, float s) {
+  const int lane = threadIdx.x & 63;
+  const bool fresh = s == 0.0f;
+  if (fresh) s = serial_sum_lds(p, 64);
+  for (int c = 0; c < m; c += kSerialStep) {
+    float v[8];
+    *(float4 *)v = ((const float4 *)(p + c))[2 * lane];
+    *(float4 *)(v + 4) = ((const float4 *)(p + c))[2 * lane + 1];
+    // zero terms leave any s >= 0 as it is
+    bool some = false;
+#pragma unroll
+    for (int j = 0; j < 8; j++) some |= !(v[j] == 0.0f);
+    if (__ballot(some) == 0) continue;
+    int l0 = fresh && c == 0 ? 8 : 0;  // lanes below l0 are in s
+    while (l0 < 64) {
+      const unsigned sb = __builtin_amdgcn_readfirstlane((int)__float_as_uint(s));
+      const int e = (int)(sb >> 23);
+      int f = l0;
+      if (e >= 27 && e <= 252) {
+        const float inv = __uint_as_float((unsigned)(277 - e) << 23), u = __uint_as_float((unsigned)(e - 23) << 23);
+        const bool on = lane >= l0;
+        float r[8], q[8];
+        bool big = false, tie = false;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+          r[j] = v[j] * inv;
+          q[j] = __builtin_rintf(r[j]);
+          big |= !(r[j] < 0x1p23f);  // a NaN too
+          tie |= fabsf(r[j] - q[j]) == 0.5f;
+        }
+        int sum = 0, ties = 0, at_tie = 0;
+        const unsigned long long tied = __ballot(on && tie && !big);
+        if (tied) {  // ties rounded down here
+#pragma unroll
+          for (int j = 0; j < 8; j++) {
+            const bool half = fabsf(r[j] - q[j]) == 0.5f;
+            q[j] = half ? floorf(r[j]) : q[j];
+            sum += (int)q[j];
+            ties += half;
+            at_tie = half ? sum : at_tie;
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < 8; j++) sum += (int)q[j];
+        }
+        if (!on || big) sum = ties = 0;
+        int inc = sum;
+        inc += SW_DPP_I(0, inc, 0x111, 0xF, true);
+        inc += SW_DPP_I(0, inc, 0x112, 0xF, true);
+        inc += SW_DPP_I(0, inc, 0x114, 0xF, true);
+        inc += SW_DPP_I(0, inc, 0x118, 0xF, true);
+        inc += SW_DPP_I(0, inc, 0x142, 0xA, false);
+        inc += SW_DPP_I(0, inc, 0x143, 0xC, false);
+        int S = (int)((sb & 0x7fffffu) | 0x800000u), excl = inc - sum;
+        if (tied) {
+          const int ft = __builtin_ctzll(tied);
+          const int odd = (S + __builtin_amdgcn_readlane(excl + at_tie, ft)) & 1;
+          inc += lane >= ft ? odd : 0;
+          excl += lane > ft ? odd : 0;
+          if (lane == ft) ties--;
+        }
+        const unsigned long long ends = __ballot(on && (big || ties > 0 || S + inc >= (1 << 24)));
+        if (ends == 0) {
+          s = (float)(S + __builtin_amdgcn_readlane(inc, 63)) * u;
+          break;
+        }
+        f = __builtin_ctzll(ends);
+        s = (float)(S + __builtin_amdgcn_readlane(excl, f)) * u;
+      }
+#pragma unroll
+      for (int j = 0; j < 8; j++) s = __fadd_rn(s, lane_value(v[j], f));
+      l0 = f + 1;
+    }
+  }
+  return s;
+}
+
 // largest unsigned value over the wave; rows a step leaves out keep 0, the
 // identity of the maximum, and lane 63 ends with the whole wave's maximum
 __device__ __forceinline__ unsigned wave_max_u32(unsigned v) {
