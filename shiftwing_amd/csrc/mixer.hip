@@ -615,13 +615,28 @@ __global__ __launch_bounds__(256) void k_gqa_prep(PrepArgs p) {
 //     values of four tiles are one float4.  The block's V values are loaded
 //     before the score MFMAs, so their latency overlaps them.
 // The waves' (m, l, O) merge in LDS in wave order; the workgroup writes
-// one partial record: O [16][HD] unnormalised, the max m [16], the sum l [16].
+// one partial record: O [16][HD] unnormalised, the max m [16], the sum l [16];
+// where every row has one split, the finished context instead (what
+// k_gqa_combine would do with one record), and nothing is left to merge.
+//
+// Splits.  One row, or rows of consecutive positions, have the same number S
+// of splits, row t on blockIdx.y.  Slot calls of several rows, which may
+// differ much in length, give every split the same number `per` of 16-key
+// blocks instead (flat): row t's workgroups are first[t] .. first[t + 1] - 1,
+// (kv head, split) in order.
+struct AttnSplits {
+  int flat, S, per;
+  int first[kMixMaxTok + 1];
+};
 struct AttnArgs {
   const float *q;  // [B][nh*hd]
   const float *k_cache, *v_cache;
   long long slot_stride;
   float *part;
-  int nh, nkv, S;
+  const float *gate;  // direct: one split a row, ctx is written here
+  float *ctx;
+  int nh, nkv, rows, direct;
+  AttnSplits sp;
   MixTok tok;
 };
 
@@ -630,17 +645,23 @@ __device__ __forceinline__ v4f mfma_f32_16x16x4(float a, float b, v4f c) {
 }
 
 constexpr int kAttnWaves = 4;  // waves of a k_gqa_attn workgroup
-template <int HD>
+template <int HD, bool FLAT>
 __global__ __launch_bounds__(64 * kAttnWaves) void k_gqa_attn(AttnArgs a) {
   constexpr int KQ = HD / 4, NT16 = HD / 16, PSZ = 16 * HD + 32;
   __shared__ float s_m[kAttnWaves][16], s_l[kAttnWaves][16];
   __shared__ float s_o[16 * (HD + 1)];  // [head][dim], rows padded
   __shared__ float s_q[16 * 4 * (HD / 4 + 4)];
-  const int t = blockIdx.y, kvh = blockIdx.x / a.S, s = blockIdx.x % a.S;
+  int t = blockIdx.y, S = a.sp.S, at = blockIdx.x;
+  if (FLAT) {
+    while (t + 1 < a.rows && (int)blockIdx.x >= a.sp.first[t + 1]) t++;
+    at -= a.sp.first[t];
+    S = (a.sp.first[t + 1] - a.sp.first[t]) / a.nkv;
+  }
+  const int kvh = at / S, s = at % S;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, n = lane & 15, kg = lane >> 4;
   const int G = a.nh / a.nkv;
   const int T = tok_pos(a.tok, t) + 1;
-  const int nb = (T + 15) / 16, per = (nb + a.S - 1) / a.S;
+  const int nb = (T + 15) / 16, per = FLAT ? a.sp.per : (nb + S - 1) / S;
   const int b0 = s * per, b1 = min(nb, b0 + per);
   const int kvrows = a.nkv * HD;
   const size_t sbase = (size_t)tok_slot(a.tok, t) * a.slot_stride + (size_t)kvh * HD;
@@ -758,7 +779,23 @@ __global__ __launch_bounds__(64 * kAttnWaves) void k_gqa_attn(AttnArgs a) {
     }
     __syncthreads();
   }
-  float *rec = a.part + ((size_t)(t * a.nkv + kvh) * a.S + s) * PSZ;
+  if (a.direct) {
+    // the divide and the sigmoid gate (c/qwen.c:3129-3134)
+    if (threadIdx.x < 16) {
+      const int h = threadIdx.x;
+      float Mh = s_m[0][h], L = 0.0f;
+      for (int w = 1; w < kAttnWaves; w++) Mh = fmaxf(Mh, s_m[w][h]);
+      for (int w = 0; w < kAttnWaves; w++)
+        if (s_m[w][h] != -INFINITY) L = __builtin_fmaf(s_l[w][h], expf(s_m[w][h] - Mh), L);
+      s_q[h] = L;
+    }
+    __syncthreads();
+    const size_t at0 = ((size_t)t * a.nh + kvh * G) * HD;
+    for (int u = threadIdx.x; u < G * HD; u += 64 * kAttnWaves)
+      a.ctx[at0 + u] = (s_o[(u / HD) * (HD + 1) + u % HD] / s_q[u / HD]) * sigmoid_ref(a.gate[at0 + u]);
+    return;
+  }
+  float *rec = a.part + (FLAT ? (size_t)blockIdx.x : (size_t)(t * a.nkv + kvh) * S + s) * PSZ;
   for (int u = threadIdx.x; u < 16 * HD; u += 64 * kAttnWaves) rec[u] = s_o[(u / HD) * (HD + 1) + u % HD];
   if (threadIdx.x < 16) {
     const int h = threadIdx.x;
@@ -784,16 +821,19 @@ constexpr int kCombWaves = 4, kCombBatch = 32;
 struct CombArgs {
   const float *part, *gate;
   float *ctx;  // [B][nh*hd]
-  int nh, nkv, hd, S;
+  int nh, nkv, hd;
+  AttnSplits sp;
 };
 
+template <bool FLAT>
 __global__ __launch_bounds__(256) void k_gqa_combine(CombArgs c) {
   __shared__ float s_o[kCombWaves][64], s_m[kCombWaves], s_l[kCombWaves];
   const int hd = c.hd, dq = hd >> 6, h = blockIdx.x / dq, t = blockIdx.y;
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, j = 64 * (blockIdx.x % dq) + lane;
-  const int G = c.nh / c.nkv, kvh = h / G, n = h % G, S = c.S;
+  const int G = c.nh / c.nkv, kvh = h / G, n = h % G;
+  const int S = FLAT ? (c.sp.first[t + 1] - c.sp.first[t]) / c.nkv : c.sp.S;
   const size_t psz = (size_t)16 * hd + 32;
-  const float *base = c.part + (size_t)(t * c.nkv + kvh) * S * psz;
+  const float *base = c.part + ((size_t)(FLAT ? c.sp.first[t] : t * c.nkv * S) + kvh * S) * psz;
   const size_t at = (size_t)t * c.nh * hd + (size_t)h * hd + j;
   const float g = w == 0 ? c.gate[at] : 0.0f;
   const int sl = w + kCombWaves * lane;  // this lane's split for the maximum and sum
@@ -1414,7 +1454,10 @@ struct GqaCall {
 
 template <int HD>
 void launch_attn(ColiCuda *ctx, const AttnArgs &a, int rows) {
-  k_gqa_attn<HD><<<dim3(a.nkv * a.S, rows), 64 * kAttnWaves, 0, ctx->stream>>>(a);
+  if (a.sp.flat)
+    k_gqa_attn<HD, true><<<a.sp.first[rows], 64 * kAttnWaves, 0, ctx->stream>>>(a);
+  else
+    k_gqa_attn<HD, false><<<dim3(a.nkv * a.sp.S, rows), 64 * kAttnWaves, 0, ctx->stream>>>(a);
 }
 
 int gqa_run(ColiCuda *ctx, const GqaCall &c) {
@@ -1430,21 +1473,54 @@ int gqa_run(ColiCuda *ctx, const GqaCall &c) {
   if ((hd != 64 && hd != 128 && hd != 256) || c.nh / c.nkv > 16 || c.rd > hd || (c.rd & 1))
     return fail_arg("%s: head_dim must be 64, 128 or 256 with at most 16 query heads per kv head", c.name);
   if (((uintptr_t)c.x & 15) || (H % 4)) return fail_arg("%s: activations must be 16-byte aligned", c.name);
-  // key splits: about 256 workgroups in all, each split at least one 16-key
-  // block per wave
-  const int T = c.max_pos + 1;
-  const int nb = (T + 15) / 16;
-  int S = (256 + c.nkv * R - 1) / (c.nkv * R);
-  const int smax = (nb + kAttnWaves - 1) / kAttnWaves;
-  S = S > smax ? smax : S;
-  S = S > kMaxSplits ? kMaxSplits : S;
-  S = S < 1 ? 1 : S;
+  // key splits: as many workgroups as are resident at once (two a compute
+  // unit), each split at least one 16-key block per wave.  Thirteen rows of 460
+  // to 6,000 keys: attention 57 us with splits sized by the longest row, 37 so
+  const int target = 2 * (ctx->sm_count > 0 ? ctx->sm_count : 256);
+  AttnSplits sp;
+  memset(&sp, 0, sizeof(sp));
+  int wgs = 0, most = 1;  // workgroups; splits of the longest row
+  if (c.tok.tab && R > 1) {
+    sp.flat = 1;
+    long long blocks = 0;
+    int longest = 0;
+    for (int r = 0; r < R; r++) {
+      const int nb = c.tok.pos[r] / 16 + 1;
+      blocks += nb;
+      longest = nb > longest ? nb : longest;
+    }
+    long long per = (blocks * c.nkv + target - 1) / target;
+    if (per < kAttnWaves) per = kAttnWaves;
+    if (per < (longest + kMaxSplits - 1) / kMaxSplits) per = (longest + kMaxSplits - 1) / kMaxSplits;
+    // the rows' last splits are partly filled: a little longer ones until all fit
+    for (;; per++) {
+      long long n = 0;
+      for (int r = 0; r < R; r++) n += (c.tok.pos[r] / 16 + per) / per;
+      if (n * c.nkv <= target || per >= longest) break;
+    }
+    sp.per = (int)per;
+    for (int r = 0; r < R; r++) {
+      const int n = (c.tok.pos[r] / 16 + sp.per) / sp.per;  // ceil of the row's blocks
+      sp.first[r] = wgs;
+      wgs += n * c.nkv;
+      most = n > most ? n : most;
+    }
+    sp.first[R] = wgs;
+  } else {
+    const int nb = c.max_pos / 16 + 1;
+    int S = target / (c.nkv * R);
+    const int smax = (nb + kAttnWaves - 1) / kAttnWaves;
+    S = S > smax ? smax : S;
+    S = S > kMaxSplits ? kMaxSplits : S;
+    sp.S = most = S < 1 ? 1 : S;
+    wgs = R * c.nkv * sp.S;
+  }
   const size_t psz = (size_t)16 * hd + 32;
   const size_t ox = 0, oqp = ox + align_up((size_t)R * H * 4), ok = oqp + align_up((size_t)R * qrows * 4),
                ov = ok + align_up((size_t)R * kvrows * 4), oq = ov + align_up((size_t)R * kvrows * 4),
                og = oq + align_up((size_t)R * ctxn * 4), oc = og + align_up((size_t)R * ctxn * 4),
                oy = oc + align_up((size_t)R * ctxn * 4), op = oy + align_up((size_t)R * H * 4),
-               od = op + align_up((size_t)R * c.nkv * S * psz * 4),
+               od = op + align_up(most > 1 ? wgs * psz * 4 : 0),
                total = od + align_up(mix_digit_bytes(R, H > ctxn ? H : ctxn));
   if (ensure_scratch(ctx, kScrMixer, total, c.name)) return -1;
   char *w = (char *)ctx->scratch[kScrMixer];
@@ -1502,7 +1578,11 @@ int gqa_run(ColiCuda *ctx, const GqaCall &c) {
   at.part = part;
   at.nh = c.nh;
   at.nkv = c.nkv;
-  at.S = S;
+  at.rows = R;
+  at.direct = most == 1;
+  at.gate = gate;
+  at.ctx = cx;
+  at.sp = sp;
   at.tok = c.tok;
   if (hd == 256)
     launch_attn<256>(ctx, at, R);
@@ -1511,15 +1591,21 @@ int gqa_run(ColiCuda *ctx, const GqaCall &c) {
   else
     launch_attn<64>(ctx, at, R);
 
-  CombArgs cb;
-  cb.part = part;
-  cb.gate = gate;
-  cb.ctx = cx;
-  cb.nh = c.nh;
-  cb.nkv = c.nkv;
-  cb.hd = hd;
-  cb.S = S;
-  k_gqa_combine<<<dim3(c.nh * (hd / 64), R), 256, 0, ctx->stream>>>(cb);
+  if (most > 1) {
+    CombArgs cb;
+    cb.part = part;
+    cb.gate = gate;
+    cb.ctx = cx;
+    cb.nh = c.nh;
+    cb.nkv = c.nkv;
+    cb.hd = hd;
+    cb.sp = sp;
+    const dim3 grid(c.nh * (hd / 64), R);
+    if (sp.flat)
+      k_gqa_combine<true><<<grid, 256, 0, ctx->stream>>>(cb);
+    else
+      k_gqa_combine<false><<<grid, 256, 0, ctx->stream>>>(cb);
+  }
 
   ProjArgs o;
   memset(&o, 0, sizeof(o));

@@ -87,3 +87,25 @@ def test_projection_non_finite_rows(be, oracle):
     got = dev.slots_step(X, [0, 1, 2, 3], [0, 0, 0, 0])
     assert np.array_equal(got[[0, 2]], clean[[0, 2]])
     assert not np.isfinite(got[[1, 3]]).any()
+
+
+@pytest.mark.parametrize("pos", [[0, 900, 31, 63, 64, 500], [300, 300], [5, 0, 15, 16]], ids=["mixed", "equal", "short"])
+def test_gqa_slots_of_different_lengths(be, oracle, pos):
+    """Key splits of one length for all rows: rows of one to several splits in
+    one call, and calls whose rows have one split each (no merge)."""
+    from oracle import pyoracle as po
+    at = po.HostAttn(81, 256, 4, 2, 64, 32, o_fmt=4)
+    n, seq = len(pos), max(pos) + 1
+    dev = _dev_attn(be, at, seq, slots=n)
+    kc, vc = at.new_cache(seq, n)
+    rng = np.random.default_rng(82)
+    import ctypes as C
+    for host, buf in ((kc, dev.k_cache), (vc, dev.v_cache)):
+        host[:] = rng.standard_normal(host.shape)
+        be.check(be.lib.coli_cuda_upload(be.ctx, buf.p, C.c_void_p(host.ctypes.data), host.nbytes), "upload")
+    be.sync()
+    X = _x(rng, n, 256)
+    print(f"[gqa slots] positions {pos}", flush=True)
+    want = np.stack([po.oracle_attn_step(oracle, at, X[r], pos[r], kc[r], vc[r]) for r in range(n)])
+    got = dev.slots_step(X, list(range(n)), pos, device_io=True)
+    assert_close_rms(got, want, 1e-4, "output")
