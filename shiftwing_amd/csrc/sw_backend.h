@@ -30,10 +30,8 @@ namespace sw {
 enum Scratch {
   kScrSetup = 0,   // reference grouped calls: route weights on the device
   kScrHidden,      // reference grouped calls: routed hidden activations
-  kScrRouteOut,    // reference grouped calls: per-route down outputs
   kScrGate,        // reference shared-expert calls: hidden vectors, gate logits
   kScrUp,
-  kScrWeight,
   kScrXPrep,       // many-token step: activation digits, routes, buckets
   kScrRouter,      // many-token step: router logit bounds
   kScrRoutes,      // many-token step: idx / weights / buckets
