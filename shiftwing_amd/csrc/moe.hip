@@ -2575,6 +2575,28 @@ __global__ __launch_bounds__(64 * kWideWaves) void k_gateup_wide(Work w, ExpertL
   }
 }
 
+// Shared down (IDOT) of kSharedBlockTokens tokens from t0: this wave's row
+// tiles rt, rt + step, ... below rt1.
+__device__ __forceinline__ void shared_down_tiles(const Work &w, const signed char *dq, const float *ds, int rt, int rt1,
+                                                  int step, int t0) {
+  const int lane = threadIdx.x & 63, kb = lane >> 4;
+  for (; rt < rt1; rt += step) {
+    v4i c[kSharedSub] = {};
+    idot_tiles<kSharedSub>(dq, w.Ish, rt * kTileRows, 0, w.Ish / 64, w.hq, w.Ish, t0, w.T, c, lane);
+#pragma unroll
+    for (int q = 0; q < kSharedSub; q++) {
+      const int tok = t0 + 16 * q + (lane & 15);
+      if (tok < w.T) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const int row = rt * kTileRows + 4 * kb + i;
+          w.shout[(size_t)tok * w.H + row] = (float)c[q][i] * ds[row] * w.shx[tok];
+        }
+      }
+    }
+  }
+}
+
 // routed down of wide items, plus the shared expert's token chunks (IDOT) in
 // the first blocks y < shc (scheduled first, they overlap the routed work).
 // Block: kWideWaves waves x kWideDnRt row tiles of H; a 1-D grid of shc*nx
@@ -2590,23 +2612,8 @@ __global__ __launch_bounds__(64 * kWideWaves) void k_down_wide(Work w, ExpertLay
   const int lin = (int)blockIdx.x;
   if (lin < shc * nx) {  // shared down, kSharedBlockTokens tokens a block
     const int rtb = lin % nx * kWideWaves * kWideDnRt;
-    const int rt1 = min(nrt, rtb + kWideWaves * kWideDnRt);
-    const int t0 = lin / nx * kSharedBlockTokens;
-    for (int rt = rtb + wave; rt < rt1; rt += kWideWaves) {
-      v4i c[kSharedSub] = {};
-      idot_tiles<kSharedSub>(dq, w.Ish, rt * kTileRows, 0, w.Ish / 64, w.hq, w.Ish, t0, w.T, c, lane);
-#pragma unroll
-      for (int q = 0; q < kSharedSub; q++) {
-        const int tok = t0 + 16 * q + (lane & 15);
-        if (tok < w.T) {
-#pragma unroll
-          for (int i = 0; i < 4; i++) {
-            const int row = rt * kTileRows + 4 * kb + i;
-            w.shout[(size_t)tok * w.H + row] = (float)c[q][i] * ds[row] * w.shx[tok];
-          }
-        }
-      }
-    }
+    shared_down_tiles(w, dq, ds, rtb + wave, min(nrt, rtb + kWideWaves * kWideDnRt), kWideWaves,
+                      lin / nx * kSharedBlockTokens);
     return;
   }
   int chunk, slot;
@@ -2630,6 +2637,266 @@ __global__ __launch_bounds__(64 * kWideWaves) void k_down_wide(Work w, ExpertLay
         if (rt >= nrt) continue;
 #pragma unroll
         for (int r = 0; r < 4; r++) w.rout[(size_t)(p0 + tt) * w.H + rt * kTileRows + 4 * kb + r] = acc[rr][0][r];
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// 7t / 8t.  Tall items, for steps whose experts hold many tokens: an item is up
+// to kTallTokens = 64 tokens of one expert, four MFMA column sets of 16, so a
+// weight tile is read and unpacked once per 64 tokens instead of once per 16
+// (1,999 tokens, S397, 39 an expert: gate/up 1060 -> 773 us, down 666 -> 448 us;
+// empty column sets are skipped).  The arithmetic of a (row, token) is that of
+// the wide items, group by group in the same order: same bits.
+// A workgroup of 8 waves takes 16 tiles, two a wave: gate and up of one row
+// tile of I, or two row tiles of H.  Per 128-column group the item's digits
+// (4 KB a column set), their parameters and every wave's records go to one of
+// two LDS buffers by global_load_lds while the previous group is worked on, one
+// barrier a group; the bytes in flight hold no registers, so two workgroups
+// share a compute unit and one's barriers, first copies and epilogue fall into
+// the other's work (one workgroup of 16 waves and three buffers: 863 and 503
+// us).  Bound by VALU (unpacking 28 instructions a tile, 25 a column set and
+// tile, about 400 us of the gate/up) and the LDS reads beside it.
+// ---------------------------------------------------------------------------
+constexpr int kTallTokens = 64;
+constexpr int kTallWaves = 8, kTallTiles = 2 * kTallWaves, kTallBufs = 2;
+__host__ __device__ constexpr int tall_slot(int fmt) { return fmt == 4 ? 2048 + 256 : 2048; }
+__host__ __device__ constexpr int tall_buf(int fmt) { return kTallWaves * tall_slot(fmt) + 16 * 1024 + kTallTokens * 16; }
+
+// acc[c][m][r] over all groups: column set c (token 16 c + lane % 16), tile m,
+// row 4 (lane / 16) + r.  DOWN 0: tiles are gate and up of row tile rt0; 1: row
+// tiles rt0 and rt1 of down.  Token rows: rows_of[p0 + tt], or p0 + tt.
+// NC column sets hold tokens: the code of a group is straight-line.
+template <int FMT, int DOWN, int NC>
+__device__ __forceinline__ void tall_rows_nc(unsigned char *lds, const ExpertLayout &xl, int e, int rt0, int rt1, int ng,
+                                          int ld, const signed char *d1, const signed char *d2, const float4 *gp,
+                                          const int *rows_of, int p0, int cnt, float (&acc)[4][2][4]) {
+  constexpr int SB = tall_slot(FMT), BUF = tall_buf(FMT), DIG = kTallWaves * SB, PAR = DIG + 16 * 1024;
+  constexpr float off = FMT == 4 ? 8.0f : 4.0f;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, kb = lane >> 4;
+  auto token_row = [&](int tt) {  // tokens past the item repeat its last one
+    const int q = p0 + (tt < cnt ? tt : cnt - 1);
+    return rows_of ? rows_of[q] : q;
+  };
+  // wave w copies plane w % 4 (digit, half) of column sets w / 4 and w / 4 + 2
+  const int set = wave >> 2;
+  const signed char *dsrc[2];
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+    dsrc[i] = ((wave & 2) ? d2 : d1) + (size_t)token_row(16 * (set + 2 * i) + (lane & 15)) * ld + (wave & 1) * 64 + kb * 16;
+  const float4 *psrc = gp + (size_t)token_row(lane) * ng;
+  const unsigned char *rec0, *rec1;
+  {
+    const unsigned char *x = xl.base + (size_t)e * xl.expert_bytes;
+    if (DOWN) {
+      rec0 = x + xl.gu_bytes + (size_t)rt0 * ng * xl.rec_d();
+      rec1 = x + xl.gu_bytes + (size_t)rt1 * ng * xl.rec_d();
+    } else {
+      rec0 = rec1 = x + (size_t)rt0 * ng * xl.rec_gu();
+    }
+  }
+  const unsigned rs = DOWN ? xl.rec_d() : xl.rec_gu();
+  auto copy = [&](int g) {
+    unsigned char *const buf = lds + (g % kTallBufs) * BUF;
+    unsigned char *const slot = buf + wave * SB;
+    const unsigned char *const a = rec0 + (size_t)g * rs, *const b = rec1 + (size_t)g * rs;
+    if (NC > 1 || set < NC) dma_b128(dsrc[0] + (size_t)g * kGroup, lds_addr(buf + DIG + wave * 1024));
+    if (NC > 2 && set + 2 < NC) dma_b128(dsrc[1] + (size_t)g * kGroup, lds_addr(buf + DIG + (wave + 8) * 1024));
+    if (wave == 0) dma_b128(psrc + g, lds_addr(buf + PAR));
+    // lanes past a record's end repeat its last 16 bytes
+    if (DOWN && FMT == 3) {
+      const int o = 16 * (lane < 52 ? lane : 51);
+      dma_b128(a + o, lds_addr(slot));
+      dma_b128(b + o, lds_addr(slot + 1024));
+    } else if (DOWN) {
+      dma_b128(a + 16 * lane, lds_addr(slot));
+      dma_b128(b + 16 * lane, lds_addr(slot + 1024));
+      dma_b32((kb & 1 ? b : a) + 1024 + 4 * (lane & 15), lds_addr(slot + 2048));
+    } else if (FMT == 3) {
+      dma_b128(a + 16 * lane, lds_addr(slot));
+      dma_b128(a + 1024 + 16 * (lane < 40 ? lane : 39), lds_addr(slot + 1024));
+    } else {
+      dma_b128(a + 16 * lane, lds_addr(slot));
+      dma_b128(a + 1024 + 16 * lane, lds_addr(slot + 1024));
+      dma_b32(a + 2048 + 4 * (lane & 31), lds_addr(slot + 2048));
+    }
+  };
+  copy(0);
+  for (int g = 0; g < ng; g++) {
+    // this group's copies are done; past the barrier every wave has left the
+    // buffer that the next copies fill
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (g + 1 < ng) copy(g + 1);
+    const unsigned char *const buf = lds + (g % kTallBufs) * BUF;
+    const unsigned char *const slot = buf + wave * SB;
+    v4i a0[2], a1[2];
+    float4 sc[2];
+#pragma unroll
+    for (int m = 0; m < 2; m++) {
+      const uint32_t *cw = (const uint32_t *)(slot + m * (FMT == 3 && !DOWN ? 768 : 1024) + lane * (FMT == 4 ? 16 : 12));
+      uint32_t q[4];
+#pragma unroll
+      for (int i = 0; i < (FMT == 4 ? 4 : 3); i++) q[i] = cw[i];
+      unpack_words<FMT>(q, a0[m], a1[m]);
+      sc[m] = *(const float4 *)(slot + (FMT == 4 ? 2048 + 64 * m : DOWN ? 1024 * m + 768 : 1536 + 64 * m) + 16 * kb);
+    }
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      const v4i *const D = (const v4i *)(buf + DIG + c * 4096);
+      const v4i b00 = D[lane], b01 = D[64 + lane], b10 = D[128 + lane], b11 = D[192 + lane];
+      const float4 pr = ((const float4 *)(buf + PAR))[16 * c + (lane & 15)];  // A, B, Q1, Q2
+      const float K = off * (pr.x * (float)__float_as_int(pr.z) + pr.y * (float)__float_as_int(pr.w));
+#pragma unroll
+      for (int m = 0; m < 2; m++) {
+        v4i c1 = {0, 0, 0, 0}, c2 = {0, 0, 0, 0};
+        c1 = mfma_i8(a0[m], b00, c1);
+        c2 = mfma_i8(a0[m], b10, c2);
+        c1 = mfma_i8(a1[m], b01, c1);
+        c2 = mfma_i8(a1[m], b11, c2);
+        const float scv[4] = {sc[m].x, sc[m].y, sc[m].z, sc[m].w};
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const float f = __builtin_fmaf(pr.x, (float)c1[r], __builtin_fmaf(pr.y, (float)c2[r], -K));
+          acc[c][m][r] = __builtin_fmaf(f, scv[r], acc[c][m][r]);
+        }
+      }
+    }
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the buffers are free
+}
+
+template <int FMT, int DOWN>
+__device__ __forceinline__ void tall_rows(unsigned char *lds, const ExpertLayout &xl, int e, int rt0, int rt1, int ng,
+                                          int ld, const signed char *d1, const signed char *d2, const float4 *gp,
+                                          const int *rows_of, int p0, int cnt, float (&acc)[4][2][4]) {
+  if (cnt > 48)
+    tall_rows_nc<FMT, DOWN, 4>(lds, xl, e, rt0, rt1, ng, ld, d1, d2, gp, rows_of, p0, cnt, acc);
+  else if (cnt > 32)
+    tall_rows_nc<FMT, DOWN, 3>(lds, xl, e, rt0, rt1, ng, ld, d1, d2, gp, rows_of, p0, cnt, acc);
+  else if (cnt > 16)
+    tall_rows_nc<FMT, DOWN, 2>(lds, xl, e, rt0, rt1, ng, ld, d1, d2, gp, rows_of, p0, cnt, acc);
+  else
+    tall_rows_nc<FMT, DOWN, 1>(lds, xl, e, rt0, rt1, ng, ld, d1, d2, gp, rows_of, p0, cnt, acc);
+}
+
+// grid nx = ceil(I/16 / 8) chunks x ny item slots (xcd_block), 512 threads, two
+// tall_buf of LDS.  A workgroup's 8 row tiles are one 128-value group of I,
+// whose digits it forms as k_gateup_wide does.
+template <int FMT>
+__global__ __launch_bounds__(64 * kTallWaves) __attribute__((amdgpu_waves_per_eu(4))) void k_gateup_tall(Work w, ExpertLayout xl, int nx, int ny) {
+  extern __shared__ __align__(16) unsigned char tlds[];
+  float(*const s_amax)[kTallTokens] = (float(*)[kTallTokens])tlds;  // [wave][token]
+  int(*const s_q)[2][kTallTokens] = (int(*)[2][kTallTokens])(tlds + kTallWaves * kTallTokens * 4);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, kb = lane >> 4, tt = lane & 15;
+  const int nrt = w.I / kTileRows;
+  int chunk, slot;
+  xcd_block((int)blockIdx.x, nx, ny, chunk, slot);
+  const int rt = chunk * kTallWaves + wave, g = chunk;  // one 128-value group of I
+  const int n_items = *w.nitems;
+  for (int it = slot; it < n_items; it += ny) {
+    const int4 item = w.items[it];
+    const int p0 = item.y, cnt = item.z, nc = (cnt + 15) / 16;
+    float acc[4][2][4] = {};
+    tall_rows<FMT, 0>(tlds, xl, item.x, rt < nrt ? rt : nrt - 1, 0, w.ngh, w.Hp, w.xd1, w.xd2, w.xgp, w.btok, p0, cnt,
+                      acc);
+    float h[4][4];
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+      if (c < nc) {
+        float m = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          h[c][r] = rt < nrt ? silu_ref(acc[c][0][r]) * acc[c][1][r] : 0.0f;
+          m = fmaxf(m, fabsf(h[c][r]));
+        }
+        m = fmaxf(m, __shfl_xor(m, 16, 64));
+        m = fmaxf(m, __shfl_xor(m, 32, 64));
+        if (kb == 0) s_amax[wave][16 * c + tt] = m;
+      }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+      if (c < nc) {
+        const int tok = 16 * c + tt;
+        float amax = 0.0f;
+#pragma unroll
+        for (int v = 0; v < 8; v++) amax = fmaxf(amax, s_amax[v][tok]);
+        const float A = amax / 127.0f, B = A / 254.0f;
+        int q1[4] = {0, 0, 0, 0}, q2[4] = {0, 0, 0, 0};
+        if (amax > 0.0f) {
+          const float invA = 127.0f / amax, invB = 254.0f / A;
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            q1[r] = (int)fminf(fmaxf(__builtin_rintf(h[c][r] * invA), -127.0f), 127.0f);
+            const float rr = __builtin_fmaf(-(float)q1[r], A, h[c][r]);
+            q2[r] = (int)fminf(fmaxf(__builtin_rintf(rr * invB), -127.0f), 127.0f);
+          }
+        }
+        const size_t at = (size_t)(p0 + tok) * w.Ip + (size_t)g * kGroup + (size_t)wave * kTileRows + 4 * kb;
+        if (tok < cnt) {
+          *(unsigned *)(w.hd1 + at) = pack_i8x4(q1[0], q1[1], q1[2], q1[3]);
+          *(unsigned *)(w.hd2 + at) = pack_i8x4(q2[0], q2[1], q2[2], q2[3]);
+        }
+        int Q1 = q1[0] + q1[1] + q1[2] + q1[3], Q2 = q2[0] + q2[1] + q2[2] + q2[3];
+        Q1 += __shfl_xor(Q1, 16, 64);
+        Q1 += __shfl_xor(Q1, 32, 64);
+        Q2 += __shfl_xor(Q2, 16, 64);
+        Q2 += __shfl_xor(Q2, 32, 64);
+        if (kb == 0) {
+          s_q[wave][0][tok] = Q1;
+          s_q[wave][1][tok] = Q2;
+        }
+      }
+    __syncthreads();
+    if (wave == 0 && lane < cnt) {  // lane: the token
+      float amax = 0.0f;
+      int S1 = 0, S2 = 0;
+#pragma unroll
+      for (int v = 0; v < 8; v++) {
+        amax = fmaxf(amax, s_amax[v][lane]);
+        S1 += s_q[v][0][lane];
+        S2 += s_q[v][1][lane];
+      }
+      const float A = amax / 127.0f, B = A / 254.0f;
+      w.hgp[(size_t)(p0 + lane) * w.ngi + g] = make_float4(A, B, __int_as_float(S1), __int_as_float(S2));
+    }
+    __syncthreads();
+  }
+}
+
+// routed down of tall items, after the shared expert's token chunks as in
+// k_down_wide; grid shc*nx + nx = ceil(H/16 / 16) chunks x ny item slots.
+template <int FMT>
+__global__ __launch_bounds__(64 * kTallWaves) __attribute__((amdgpu_waves_per_eu(4))) void k_down_tall(Work w, ExpertLayout xl, int shc, const signed char *dq,
+                                                               const float *ds, int nx, int ny) {
+  extern __shared__ __align__(16) unsigned char tlds[];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, kb = lane >> 4;
+  const int nrt = w.H / kTileRows, lin = (int)blockIdx.x;
+  if (lin < shc * nx) {
+    shared_down_tiles(w, dq, ds, lin % nx * kTallTiles + wave, min(nrt, (lin % nx + 1) * kTallTiles), kTallWaves,
+                      lin / nx * kSharedBlockTokens);
+    return;
+  }
+  int chunk, slot;
+  xcd_block(lin - shc * nx, nx, ny, chunk, slot);
+  const int rt0 = chunk * kTallTiles + 2 * wave;
+  const int n_items = *w.nitems;
+  for (int it = slot; it < n_items; it += ny) {
+    const int4 item = w.items[it];
+    const int p0 = item.y, cnt = item.z;
+    float acc[4][2][4] = {};
+    tall_rows<FMT, 1>(tlds, xl, item.x, rt0 < nrt ? rt0 : nrt - 1, rt0 + 1 < nrt ? rt0 + 1 : nrt - 1, w.ngi, w.Ip,
+                      w.hd1, w.hd2, w.hgp, nullptr, p0, cnt, acc);
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      const int tok = 16 * c + (lane & 15);
+      if (tok < cnt) {
+#pragma unroll
+        for (int m = 0; m < 2; m++)
+          if (rt0 + m < nrt)
+            *(float4 *)(w.rout + (size_t)(p0 + tok) * w.H + (rt0 + m) * kTileRows + 4 * kb) =
+                make_float4(acc[c][m][0], acc[c][m][1], acc[c][m][2], acc[c][m][3]);
       }
     }
   }
@@ -3103,18 +3370,24 @@ static int route_launch(ColiCuda *ctx, ColiMoeLayer *L, Work &w, const float *x)
 // no block barrier, and are faster at every step size measured, however few
 // tokens an expert holds (S397: 834 against 686 tok/s at 8 tokens a step,
 // 1763 against 1388 at 32).  The context's setting
-// (coli_cuda_moe_set_item_tokens) can force either.
-static int item_tokens(const ColiCuda *ctx, const ColiMoeLayer *L) {
+// (coli_cuda_moe_set_item_tokens) can force either.  Tall items from
+// kTallMinTokens tokens an expert on average, against wide ones: S397 at 10 / 16 /
+// 20 / 39 tokens an expert 992 / 1122 / 1289 / 1978 against 920 / 1180 / 1489 / 2389
+// us a step, S35 at 16 / 20 / 32 / 47 270 / 304 / 396 / 463 against 255 / 310 / 422 /
+// 517.
+constexpr int kTallMinTokens = 18;
+static int item_tokens(const ColiCuda *ctx, const ColiMoeLayer *L, int T) {
   const int mode = ctx->moe_item_tokens;
   const bool fits = wide_lds_bytes(wide_stage_groups(L->ngh, kWideGuBatch)) <= 160 * 1024 &&
                     wide_lds_bytes(wide_stage_groups(L->ngi, kWideDnBatch)) <= 160 * 1024;
+  if (mode == 0 && (long long)T * L->sh.topk >= (long long)kTallMinTokens * L->sh.experts) return kTallTokens;
   return fits && mode != kMaxTokensPerItem ? kWideTokens : kMaxTokensPerItem;
 }
 
 static int prepare(ColiCuda *ctx, ColiMoeLayer *L, int T, Work &w) {
   if (T <= 0 || T > kMaxTokens) return fail_arg("MoE step: tokens %d outside [1,%d]", T, kMaxTokens);
   w = make_work(L, T);
-  w.itok = item_tokens(ctx, L);
+  w.itok = item_tokens(ctx, L, T);
   size_t bytes = carve(w, nullptr);
   if (ensure_scratch(ctx, kScrXPrep, bytes, "MoE workspace allocation")) return -1;
   carve(w, (char *)ctx->scratch[kScrXPrep]);
@@ -3228,7 +3501,18 @@ extern "C" int coli_cuda_moe_forward(ColiCuda *ctx, ColiMoeLayer *L, float *y, c
   if (slots > 1024) slots = 1024;
   const bool fmt4 = L->sh.expert_format == 4;
   const bool wide_items = w.itok > kMaxTokensPerItem;
-  if (wide_items) {
+  const bool tall_items = w.itok == kTallTokens;
+  if (tall_items) {
+    k_prep_hidden<<<T, 256, 0, st>>>(w, L->sh_gs, L->sh_us);  // the shared hidden rows
+    const int nx = (w.I / kTileRows + kTallWaves - 1) / kTallWaves;
+    const void *fn = fmt4 ? (const void *)k_gateup_tall<4> : (const void *)k_gateup_tall<3>;
+    const size_t lds = (size_t)kTallBufs * tall_buf(fmt4 ? 4 : 3);
+    if (set_lds(fn, lds)) return -1;
+    if (fmt4)
+      k_gateup_tall<4><<<nx * slots, 64 * kTallWaves, lds, st>>>(w, L->xl, nx, slots);
+    else
+      k_gateup_tall<3><<<nx * slots, 64 * kTallWaves, lds, st>>>(w, L->xl, nx, slots);
+  } else if (wide_items) {
     const int hg = wide_stage_groups(w.ngh, kWideGuBatch);
     const size_t lg = wide_lds_bytes(hg);
     const void *fn = fmt4 ? (const void *)k_gateup_wide<4> : (const void *)k_gateup_wide<3>;
@@ -3268,7 +3552,17 @@ extern "C" int coli_cuda_moe_forward(ColiCuda *ctx, ColiMoeLayer *L, float *y, c
   const int dn_blocks_x = (w.H / kTileRows + 4 * kDnRowTiles - 1) / (4 * kDnRowTiles);
   const bool dn_split = w.ngi <= 8;
   const int ds_blocks_x = (w.H / kTileRows + kDnBlockRows - 1) / kDnBlockRows;
-  if (wide_items) {
+  if (tall_items) {
+    const int shc = (T + kSharedBlockTokens - 1) / kSharedBlockTokens;
+    const int nx = (w.H / kTileRows + kTallTiles - 1) / kTallTiles;
+    const void *fn = fmt4 ? (const void *)k_down_tall<4> : (const void *)k_down_tall<3>;
+    const size_t lds = (size_t)kTallBufs * tall_buf(fmt4 ? 4 : 3);
+    if (set_lds(fn, lds)) return -1;
+    if (fmt4)
+      k_down_tall<4><<<nx * (shc + slots), 64 * kTallWaves, lds, st>>>(w, L->xl, shc, L->sh_dq, L->sh_ds, nx, slots);
+    else
+      k_down_tall<3><<<nx * (shc + slots), 64 * kTallWaves, lds, st>>>(w, L->xl, shc, L->sh_dq, L->sh_ds, nx, slots);
+  } else if (wide_items) {
     const int hg = wide_stage_groups(w.ngi, kWideDnBatch);
     const size_t ld = wide_lds_bytes(hg);
     const void *fn = fmt4 ? (const void *)k_down_wide<4> : (const void *)k_down_wide<3>;
