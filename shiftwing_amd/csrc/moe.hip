@@ -654,58 +654,93 @@ __device__ __forceinline__ double gemm_bound_factor(int H) {
   return (n * u / (1.0 - n * u) + n * v / (1.0 - n * v)) * (1.0 + 0x1p-20);
 }
 
-// One 16-token x 16-row tile of L per block; its 4 waves take a quarter of
-// the k range each and their sums meet in LDS in wave order.  MFMA step c of
-// k block kb pairs x_t[16 kb + 4 (l >> 4) + c] with w_e[16 kb + 4 (l >> 4) +
-// c] at lane l (A: token t0 + l % 16, B: row e0 + l % 16), so every lane
+// NT x NT tiles of 16 tokens x 16 rows of L per block; its 4 waves take a
+// quarter of the k range each and their sums meet in LDS in wave order.  MFMA
+// step c of k block kb pairs x_t[16 kb + 4 (l >> 4) + c] with w_e[16 kb + 4 (l >>
+// 4) + c] at lane l (A: token t0 + l % 16, B: row e0 + l % 16), so every lane
 // loads float4s; the result holds token t0 + (l >> 4) + 4 v, row e0 + l % 16
 // at lane l, item v (the f64 16x16x4 output layout: D[(l >> 4) + 4 v][l % 16]).
-// The same loads give ||x_t|| and ||w_e|| (fp64 sums of squares).
-// grid (ceil(E/16), ceil(T/16)), 256 threads.  H % 64 == 0, x 16-byte aligned.
+// The same loads give ||x_t|| and ||w_e|| (fp64 sums of squares).  NT 1 waits
+// on its loads from L2; NT 2 halves them, where the blocks still fill the
+// device (1,999 tokens, S397: 276 -> 185 us; the MFMAs alone 107 us).
+// grid (ceil(E/(16 NT)), ceil(T/(16 NT))), 256 threads.  H % 64 == 0, x
+// 16-byte aligned.
+template <int NT>
 __global__ __launch_bounds__(256) void k_router_gemm(Work w, const float *x, const float *router) {
-  __shared__ double s_acc[4][4][64];
-  __shared__ double s_nx[4][64], s_nw[4][64];
+  __shared__ double s_acc[4][NT][NT][4][64];
+  __shared__ double s_nx[4][NT][64], s_nw[4][NT][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int t0 = blockIdx.y * 16, e0 = blockIdx.x * 16;
+  const int t0 = blockIdx.y * 16 * NT, e0 = blockIdx.x * 16 * NT;
   const int H = w.H, kq = H / 4;
-  const int ta = min(t0 + (lane & 15), w.T - 1), eb = min(e0 + (lane & 15), w.E - 1);
-  const float *xa = x + (size_t)ta * H + wave * kq + 4 * (lane >> 4);
-  const float *wb = router + (size_t)eb * H + wave * kq + 4 * (lane >> 4);
-  v4d acc = {0.0, 0.0, 0.0, 0.0};
-  double qa = 0.0, qb = 0.0;
-#pragma unroll 4
+  const float *xa[NT], *wb[NT];
+#pragma unroll
+  for (int i = 0; i < NT; i++) {
+    const int ta = min(t0 + 16 * i + (lane & 15), w.T - 1), eb = min(e0 + 16 * i + (lane & 15), w.E - 1);
+    xa[i] = x + (size_t)ta * H + wave * kq + 4 * (lane >> 4);
+    wb[i] = router + (size_t)eb * H + wave * kq + 4 * (lane >> 4);
+  }
+  v4d acc[NT][NT];
+  double qa[NT], qb[NT];
+#pragma unroll
+  for (int i = 0; i < NT; i++) {
+    qa[i] = qb[i] = 0.0;
+#pragma unroll
+    for (int j = 0; j < NT; j++) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
+  }
+#pragma unroll(4 / NT)
   for (int k = 0; k < kq; k += 16) {
-    const float4 a = *(const float4 *)(xa + k), b = *(const float4 *)(wb + k);
-    const double a0 = a.x, a1 = a.y, a2 = a.z, a3 = a.w, b0 = b.x, b1 = b.y, b2 = b.z, b3 = b.w;
-    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a2, b2, acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a3, b3, acc, 0, 0, 0);
-    qa = __builtin_fma(a0, a0, __builtin_fma(a1, a1, __builtin_fma(a2, a2, __builtin_fma(a3, a3, qa))));
-    qb = __builtin_fma(b0, b0, __builtin_fma(b1, b1, __builtin_fma(b2, b2, __builtin_fma(b3, b3, qb))));
+    double av[NT][4], bv[NT][4];
+#pragma unroll
+    for (int i = 0; i < NT; i++) {
+      const float4 a = *(const float4 *)(xa[i] + k), b = *(const float4 *)(wb[i] + k);
+      av[i][0] = a.x, av[i][1] = a.y, av[i][2] = a.z, av[i][3] = a.w;
+      bv[i][0] = b.x, bv[i][1] = b.y, bv[i][2] = b.z, bv[i][3] = b.w;
+    }
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+#pragma unroll
+      for (int i = 0; i < NT; i++)
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i][c], bv[j][c], acc[i][j], 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < NT; i++)
+#pragma unroll
+      for (int c = 3; c >= 0; c--) {
+        qa[i] = __builtin_fma(av[i][c], av[i][c], qa[i]);
+        qb[i] = __builtin_fma(bv[i][c], bv[i][c], qb[i]);
+      }
   }
   // sums of squares: lanes l, l^16, l^32, l^48 share a token / a row
-  qa += __shfl_xor(qa, 16, 64);
-  qa += __shfl_xor(qa, 32, 64);
-  qb += __shfl_xor(qb, 16, 64);
-  qb += __shfl_xor(qb, 32, 64);
 #pragma unroll
-  for (int v = 0; v < 4; v++) s_acc[wave][v][lane] = acc[v];
-  s_nx[wave][lane] = qa;
-  s_nw[wave][lane] = qb;
+  for (int i = 0; i < NT; i++) {
+    qa[i] += __shfl_xor(qa[i], 16, 64);
+    qa[i] += __shfl_xor(qa[i], 32, 64);
+    qb[i] += __shfl_xor(qb[i], 16, 64);
+    qb[i] += __shfl_xor(qb[i], 32, 64);
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) s_acc[wave][i][j][v][lane] = acc[i][j][v];
+    s_nx[wave][i][lane] = qa[i];
+    s_nw[wave][i][lane] = qb[i];
+  }
   __syncthreads();
-  if (wave != 0) return;
-  const int e = e0 + (lane & 15);
-  if (e >= w.E) return;
-  const double nw = sqrt(((s_nw[0][lane] + s_nw[1][lane]) + s_nw[2][lane]) + s_nw[3][lane]);
-  const double f = gemm_bound_factor(H) * nw;
+  for (int ij = wave; ij < NT * NT; ij += 4) {  // a wave finishes a tile
+    const int ti = ij / NT, tj = ij % NT;
+    const int e = e0 + 16 * tj + (lane & 15);
+    if (e >= w.E) continue;
+    const double nw = sqrt(((s_nw[0][tj][lane] + s_nw[1][tj][lane]) + s_nw[2][tj][lane]) + s_nw[3][tj][lane]);
+    const double f = gemm_bound_factor(H) * nw;
 #pragma unroll
-  for (int v = 0; v < 4; v++) {
-    const int i = (lane >> 4) + 4 * v, t = t0 + i;
-    if (t >= w.T) continue;
-    const double L = ((s_acc[0][v][lane] + s_acc[1][v][lane]) + s_acc[2][v][lane]) + s_acc[3][v][lane];
-    const double nx = sqrt(((s_nx[0][i] + s_nx[1][i]) + s_nx[2][i]) + s_nx[3][i]);
-    w.lb[(size_t)t * (w.E + 1) + e] = make_double2(L, f * nx + 1e-36);
+    for (int v = 0; v < 4; v++) {
+      const int i = (lane >> 4) + 4 * v, t = t0 + 16 * ti + i;
+      if (t >= w.T) continue;
+      const double L = ((s_acc[0][ti][tj][v][lane] + s_acc[1][ti][tj][v][lane]) + s_acc[2][ti][tj][v][lane]) +
+                       s_acc[3][ti][tj][v][lane];
+      const double nx = sqrt(((s_nx[0][ti][i] + s_nx[1][ti][i]) + s_nx[2][ti][i]) + s_nx[3][ti][i]);
+      w.lb[(size_t)t * (w.E + 1) + e] = make_double2(L, f * nx + 1e-36);
+    }
   }
 }
 
@@ -1165,9 +1200,12 @@ __device__ void topk_check_token(Work &w, int t, unsigned long long *stats) {
 // with coalesced loads into LDS, then one lane runs the serial sum over LDS,
 // s = rn(s + p_i), and the fused tail.  Same result as exact_chain.
 // Blocks walk the list of uncertain tokens (few: most launches find none).
-// grid (64, kUncertainSlots), 64 threads, dynamic LDS 4*H bytes.
+// grid (kUncertainChains, min(T, kUncertainSlots)), 64 threads, dynamic LDS
+// 4*H bytes: a token's set holds little more than K experts, and 1,999 tokens
+// leave some 150 uncertain (64 x 128 blocks walked them in two rounds, 110 us
+// at S397, 26 us for the 512 tokens of an S35 chunk; 16 x 512 90 and 17 us).
 // ---------------------------------------------------------------------------
-constexpr int kUncertainSlots = 128;
+constexpr int kUncertainChains = 16, kUncertainSlots = 512;
 __global__ __launch_bounds__(64) void k_exact_logits(Work w, const float *x, const float *router,
                                                      unsigned long long *stats) {
   extern __shared__ float prod[];
@@ -3303,6 +3341,9 @@ static void certify_launch(ColiCuda *ctx, ColiMoeLayer *L, Work &w, const float 
                                                                                        L->sgate_row);
 }
 
+// Blocks of 32 x 32 from which k_router_gemm<2> is the faster: 1,008 (1,999
+// tokens, S397) 185 against 276 us, 128 (512 tokens, S35) 35 against 24.
+constexpr int kRouterGemm2Blocks = 384;
 static int route_launch(ColiCuda *ctx, ColiMoeLayer *L, Work &w, const float *x) {
   hipStream_t st = ctx->stream;
   // the tiled bounds kernel resets the certification counters and the
@@ -3341,7 +3382,11 @@ static int route_launch(ColiCuda *ctx, ColiMoeLayer *L, Work &w, const float *x)
     else
       k_prep_x_any<<<w.T, 1024, 0, st>>>(w, x, L->sgate_row);
     if (w.T >= kRouterGemmTokens && w.H % 64 == 0 && ((uintptr_t)x & 15) == 0) {
-      k_router_gemm<<<dim3((w.E + 15) / 16, (w.T + 15) / 16), 256, 0, st>>>(w, x, L->router);
+      const int b2 = (w.E + 31) / 32 * ((w.T + 31) / 32);
+      if (b2 >= kRouterGemm2Blocks)
+        k_router_gemm<2><<<dim3((w.E + 31) / 32, (w.T + 31) / 32), 256, 0, st>>>(w, x, L->router);
+      else
+        k_router_gemm<1><<<dim3((w.E + 15) / 16, (w.T + 15) / 16), 256, 0, st>>>(w, x, L->router);
       k_router_refine<<<w.T, 256, (size_t)64 * (w.H / 64 + 1) * 4, st>>>(w, x, L->router);
     } else {
       k_router_bounds<<<dim3((w.E + 3) / 4, w.T), 256, 0, st>>>(w, x, L->router);
@@ -3354,7 +3399,7 @@ static int route_launch(ColiCuda *ctx, ColiMoeLayer *L, Work &w, const float *x)
       k_certify<<<w.T, 512, 0, st>>>(w, L->router_mode, L->stats);
   }
   if (set_lds((const void *)k_exact_logits, (size_t)w.H * 4)) return -1;
-  k_exact_logits<<<dim3(64, w.T < kUncertainSlots ? w.T : kUncertainSlots), 64, (size_t)w.H * 4, st>>>(
+  k_exact_logits<<<dim3(kUncertainChains, w.T < kUncertainSlots ? w.T : kUncertainSlots), 64, (size_t)w.H * 4, st>>>(
       w, x, L->router, L->stats);
   const int e4 = (w.E + 3) & ~3;
   const size_t full_lds = (size_t)4 * (w.H > 2 * e4 ? w.H : 2 * e4);
