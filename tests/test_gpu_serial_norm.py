@@ -3,7 +3,7 @@ runs of integer adds within one binade on the device; rows made to hit every
 way a run ends must still equal the serial chain bit for bit: ties (squares
 that lie halfway between two values of the running sum), many binade steps,
 terms larger than the sum, zeros, sums below and above the exactly scaled
-range, infinities and NaN, and lengths around the 64-term start, the 256-term
+range, infinities and NaN, and lengths around the 64-term start, the 512-term
 step and the 4,096-term chunk."""
 import numpy as np
 import pytest
@@ -41,7 +41,7 @@ def _rows(rng, n):
     yield "nan", y
 
 
-@pytest.mark.parametrize("n", [1, 63, 64, 65, 255, 256, 257, 2048, 4095, 4096, 4097, 9000])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 511, 512, 513, 2048, 4095, 4096, 4097, 9000])
 def test_serial_sum_of_squares(be, oracle, n):
     rng = np.random.default_rng(n)
     names, rows = zip(*_rows(rng, n))
