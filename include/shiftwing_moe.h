@@ -175,7 +175,10 @@ int coli_cuda_shared_q4_mlp_f16(
  * *_device forms (which do not synchronize); slot and position tables are
  * host arrays.  Arithmetic is fp32 on fp32 activations (the reference rounds
  * them to fp16 first) and matches the reference CPU path (gdn_forward
- * c/qwen.c:3005, attn_forward 3094) within 1e-3 x RMS.  Layouts taken: int4
+ * c/qwen.c:3005, attn_forward 3094) within 1e-3 x RMS.  Calls of several
+ * tokens may form a projection's products as exact integers; whatever the
+ * activations' range, its error stays that of fp32 sums of the row's own
+ * products, and an infinity gives a signed infinity (NaN where its code is 0).  Layouts taken: int4
  * projections with group sizes and widths that are multiples of 32 and row
  * strides that are multiples of 16 bytes (the converter's g128 rows), int8 or
  * int4 o projection, key_dim <= 128, value_dim <= 256, head_dim 64, 128 or

@@ -1173,8 +1173,7 @@ int launch_proj_mfma(ColiCuda *ctx, const ProjArgs &a, unsigned char *dig) {
   d.ldx = a.ldx;
   d.cols = a.cols;
   d.T = a.B;
-  d.dig = dig;
-  d.asc = (float *)(dig + mix_digit_scales_at(a.B, a.cols));
+  d.d = mix_digits_at(dig, a.B, a.cols);
   d.msp = a.msp;
   d.nsp = a.nsp;
   d.hw = a.hw;
@@ -1199,8 +1198,7 @@ int launch_proj_mfma(ColiCuda *ctx, const ProjArgs &a, unsigned char *dig) {
   f.tiles = nt;
   f.G = a.cols / 128;
   f.T = a.B;
-  f.dig = dig;
-  f.asc = d.asc;
+  f.d = d.d;
   if (CONV) {
     f.conv_state = a.conv_state;
     f.conv_w = a.conv_w;

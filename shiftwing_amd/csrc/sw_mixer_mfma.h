@@ -3,18 +3,32 @@
 //   y[t][row] = sum_g s[row][g] * sum_{i in g} code(row, i) * x[t][i]
 //
 // over int4 rows in groups of 128 or int8 rows with one scale, fp32
-// activations.  Each 128-column group of a token's activations is held as a
-// 30-bit fixed-point number: q = rint(x * 2^k) with 2^k the power of two that
-// brings the group's largest magnitude into [2^29, 2^30), so every value
-// within 2^-6 of that largest one is exact and the others are off by at most
-// 2^-31 of it (less than one fp32 rounding of the group's sum).  q is cut
-// into four balanced base-256 digits, each an MFMA B operand; the four int32
-// dots with the (small, exact) weight codes are exact, and are put together
-// as ((c1 * 256 + c2) * 2^16 + (c3 * 256 + c4)) * 2^-k in fp32: one rounding
-// for the group, then one FMA with the row's group scale.
+// activations.  Each 128-column group of a token's activations is held as
+// 30-bit fixed-point numbers q = rint(x * 2^k), 2^k the power of two that
+// brings the largest magnitude among them into [2^29, 2^30).  q is cut into
+// four balanced base-256 digits, each an MFMA B operand; the four int32 dots
+// with the (small, exact) weight codes are exact, and are put together in fp32
+// as (c1 * 256 + c2) * 2^16 + (c3 * 256 + c4), times 2^-k (exact): three
+// roundings for the group (both conversions and the FMA), then one FMA with
+// the row's group scale.
+//
+// A value is exact down to 2^-6 of the largest and off by at most 2^-31 of the
+// largest below.  That is less than the roundings of an fp32 sum as long as
+// the group's larger values are several, since then every row's sum has terms of
+// their size: with eight values that are at least 2^-6 of the largest, the
+// others' errors (112 of them, codes of RMS 4.6) come to 6.5e-8 of the sum of
+// a row whose code is 0 for the largest, where an fp32 chain of the group is
+// 1.1e-7 off.  So a leading range (within 2^-5 of the largest's binade) of
+// fewer than kDigBulk values that would cost the rest any bit leaves the
+// digits, the next range is tried, and what left (outliers, an infinity, a
+// NaN, all of a group below 2^-91) is added column by column by fp32 FMAs.
+// With it the error of a row follows the sum of its own terms' magnitudes,
+// whatever else the group holds: one value of 1e6 among N(0, 1), rows with the
+// code 0 there, 2.8e-4 of the sum without, 1e-7 so.  Groups of N(0, 1) values
+// and the layers' own activations hardly ever have such a column.
 //
 // k_mix_digits forms the digits once per call in the MFMA's own lane order;
-// k_mix_mfma streams the weights.
+// k_mix_mfma and k_mix_gemm run the weights against them.
 #pragma once
 
 #include "sw_device.h"
@@ -25,20 +39,55 @@ namespace sw {
 constexpr int kDigPlanes = 8;  // four digits x two 64-column halves of a group
 constexpr int kDigTile = 16;   // tokens of one MFMA B operand
 
-// Bytes of the digits and the group scales of `tokens` rows of `cols`.
+constexpr int kDigBulk = 8;    // values a range needs to stay in the digits
+
+// What k_mix_digits leaves behind of `tokens` rows of `cols`: the digits, the
+// group scales [tile][group][16 tokens] (sign set: the token has columns
+// outside the digits), the bits of those columns [tile][group][16 tokens][128]
+// and their values [token][cols] (only those are written).
+struct MixDigits {
+  unsigned char *dig;
+  float *asc;
+  unsigned char *mask;
+  float *out;
+};
 inline size_t mix_digit_bytes(int tokens, int cols) {
-  return (size_t)((tokens + kDigTile - 1) / kDigTile) * (cols / 128) * (kDigPlanes * 1024 + kDigTile * 4);
+  const size_t units = (size_t)((tokens + kDigTile - 1) / kDigTile) * (cols / 128);
+  return units * (kDigPlanes * 1024 + kDigTile * (4 + 16 + 128 * 4));
 }
-// The group scales lie behind the digits: [tile][group][16 tokens].
-__host__ __device__ inline size_t mix_digit_scales_at(int tokens, int cols) {
-  return (size_t)((tokens + kDigTile - 1) / kDigTile) * (cols / 128) * (kDigPlanes * 1024);
+inline MixDigits mix_digits_at(unsigned char *p, int tokens, int cols) {
+  const size_t units = (size_t)((tokens + kDigTile - 1) / kDigTile) * (cols / 128);
+  MixDigits d;
+  d.dig = p;
+  d.asc = (float *)(d.dig + units * (kDigPlanes * 1024));
+  d.mask = (unsigned char *)(d.asc + units * kDigTile);
+  d.out = (float *)(d.mask + units * kDigTile * 16);
+  return d;
+}
+
+// over the 16 lanes of a DPP row, in every lane
+__device__ __forceinline__ unsigned row_max_u32(unsigned v) {
+#define SW_ROW_MAX(ctrl)                                            \
+  {                                                                 \
+    const unsigned o_ = (unsigned)SW_DPP_I(0, (int)v, ctrl, 0xF, true); \
+    v = o_ > v ? o_ : v;                                            \
+  }
+  SW_ROW_MAX(0xB1) SW_ROW_MAX(0x4E) SW_ROW_MAX(0x141) SW_ROW_MAX(0x140)
+#undef SW_ROW_MAX
+  return v;
+}
+__device__ __forceinline__ int row_sum_i32(int v) {
+  v += SW_DPP_I(0, v, 0xB1, 0xF, true);
+  v += SW_DPP_I(0, v, 0x4E, 0xF, true);
+  v += SW_DPP_I(0, v, 0x141, 0xF, true);
+  v += SW_DPP_I(0, v, 0x140, 0xF, true);
+  return v;
 }
 
 struct DigitArgs {
   const float *x;  // token t at x + t * ldx
   int ldx, cols, T;
-  unsigned char *dig;
-  float *asc;
+  MixDigits d;
   // optional per-(token, head) factor 1/sqrt(sum(msp) / hw + eps)
   const float *msp;
   int nsp, hw;
@@ -50,7 +99,7 @@ struct DigitArgs {
 // [digit d][half h][lane kb * 16 + token][16 bytes].  ROWS8 0 (int4 rows):
 // byte j of half h is column 32 kb + 2 j + h, the low (0) or high (1) nibble
 // of byte j of the 16 that a lane loads; 1 (int8 rows): column
-// 32 kb + 16 h + j.  A group with an infinity or NaN gets the scale NaN.
+// 32 kb + 16 h + j.  Columns outside the digits have the digits 0.
 // Latency-bound: 4.5 us up to 16 tokens.
 // grid (cols / 128, 4 * tiles), 64 threads.
 template <int ROWS8>
@@ -70,24 +119,46 @@ __global__ __launch_bounds__(64) void k_mix_digits(DigitArgs a) {
 #pragma unroll
     for (int e = 0; e < 8; e++) v[e] *= r;
   }
-  // magnitudes as integers: a NaN orders above infinity
-  unsigned mb = 0;
+  // magnitudes as integers; infinities and NaNs leave the digits at once
+  unsigned b[8], left = 0;
 #pragma unroll
   for (int e = 0; e < 8; e++) {
-    const unsigned b = __float_as_uint(v[e]) & 0x7fffffffu;
-    mb = b > mb ? b : mb;
+    b[e] = __float_as_uint(v[e]) & 0x7fffffffu;
+    left |= b[e] >= 0x7f800000u ? 1u << e : 0;
   }
+  unsigned mb;  // the largest in the digits
+  int k;
+  float scale;
+  for (;;) {  // each turn takes a value out of one token's digits, or is the last
+    mb = 0;
 #pragma unroll
-  for (int o = 1; o < 16; o <<= 1) {
-    const unsigned b = (unsigned)__shfl_xor((int)mb, o);
-    mb = b > mb ? b : mb;
+    for (int e = 0; e < 8; e++) mb = !(left >> e & 1) && b[e] > mb ? b[e] : mb;
+    mb = row_max_u32(mb);
+    const int E = (int)(mb >> 23), k0 = 29 + 127 - E;
+    k = k0 < 120 ? k0 : 120;
+    scale = __uint_as_float((unsigned)(k + 127) << 23);
+    // below 2^-91 the scale would leave the normal range: all of it goes out
+    const bool tiny = k0 > 120;
+    const unsigned lo = tiny ? 1 : (unsigned)(E - 5) << 23;
+    unsigned big = 0;
+#pragma unroll
+    for (int e = 0; e < 8; e++) big |= !(left >> e & 1) && b[e] >= lo ? 1u << e : 0;
+    bool drop = mb != 0 && (row_sum_i32(__builtin_popcount(big)) < kDigBulk || tiny);
+    if (__ballot(drop) == 0) break;
+    bool lossy = false;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      const float r = v[e] * scale;
+      lossy |= !(left >> e & 1) && r != __builtin_rintf(r);
+    }
+    drop = drop && (tiny || (__ballot(lossy) >> (lane & 48) & 0xffff) != 0);
+    if (__ballot(drop) == 0) break;
+    if (drop) left |= big;
   }
-  const bool bad = mb >= 0x7f800000u;
-  const int k0 = 29 + 127 - (int)(mb >> 23), k = k0 < 120 ? k0 : 120;
   unsigned d[4][2] = {};
 #pragma unroll
   for (int e = 0; e < 8; e++) {
-    int q = bad ? 0 : (int)__builtin_rintf(__builtin_ldexpf(v[e], k));
+    int q = left >> e & 1 ? 0 : (int)__builtin_rintf(v[e] * scale);
     const int w = ROWS8 ? e >> 2 : e & 1, sh = 8 * (ROWS8 ? e & 3 : e >> 1);
 #pragma unroll
     for (int p = 3; p > 0; p--) {
@@ -97,7 +168,7 @@ __global__ __launch_bounds__(64) void k_mix_digits(DigitArgs a) {
     }
     d[0][w] |= (unsigned)(q & 255) << sh;
   }
-  unsigned *const out = (unsigned *)a.dig + ((size_t)tile * G + g) * (kDigPlanes * 256) + (kb * 16 + n) * 4;
+  unsigned *const out = (unsigned *)a.d.dig + ((size_t)tile * G + g) * (kDigPlanes * 256) + (kb * 16 + n) * 4;
 #pragma unroll
   for (int p = 0; p < 4; p++)
 #pragma unroll
@@ -105,10 +176,42 @@ __global__ __launch_bounds__(64) void k_mix_digits(DigitArgs a) {
       const int half = ROWS8 ? (i & 3) >> 1 : w, dw = ROWS8 ? 2 * (i & 1) + w : i & 3;
       out[(2 * p + half) * 256 + dw] = d[p][w];
     }
+  if (t >= a.T) left = 0;  // an absent token of the tile
+  const size_t at = ((size_t)tile * G + g) * kDigTile + n;
+  a.d.mask[at * 16 + i] = (unsigned char)left;
+  if (left) {
+#pragma unroll
+    for (int e = 0; e < 8; e++)
+      if (left >> e & 1) a.d.out[(size_t)t * a.cols + col + e] = v[e];
+  }
+  const unsigned some = (unsigned)(__ballot(left != 0) >> (lane & 48)) & 0xffffu;
   // int4 codes enter the MFMA as 16 * (nibble - 8)
-  if (i == 0)
-    a.asc[((size_t)tile * G + g) * kDigTile + n] =
-        bad ? __builtin_nanf("") : mb == 0 ? 0.0f : __builtin_ldexpf(ROWS8 ? 1.0f : 0.0625f, -k);
+  if (i == 0) {
+    const float sc = mb == 0 ? 0.0f : __builtin_ldexpf(ROWS8 ? 1.0f : 0.0625f, -k);
+    a.d.asc[at] = some ? -sc : sc;
+  }
+}
+
+// The columns of one token and group that are outside the digits: their
+// products with the codes of this lane's four rows, code(e, column).
+template <class Code>
+__device__ __forceinline__ void add_left_out(const unsigned char *mask, const float *out, const v4f &s4, v4f &acc,
+                                             Code code) {
+  const uint4 m = *(const uint4 *)mask;
+  const unsigned w[4] = {m.x, m.y, m.z, m.w};
+#pragma unroll 1
+  for (int i = 0; i < 4; i++)
+    for (unsigned u = i == 0 ? w[0] : i == 1 ? w[1] : i == 2 ? w[2] : w[3]; u; u &= u - 1) {
+      const int c = 32 * i + __builtin_ctz(u);
+      const float x = out[c];
+#pragma unroll
+      for (int e = 0; e < 4; e++) acc[e] = __builtin_fmaf(code(e, c) * x, s4[e], acc[e]);
+    }
+}
+// code of column c (of a group) in its byte
+template <int FMT>
+__device__ __forceinline__ float code_of(unsigned char b, int c) {
+  return FMT == 4 ? (float)((int)((b >> (4 * (c & 1))) & 15) - 8) : (float)(signed char)b;
 }
 
 // What one token of a Gated DeltaNet call reads and writes in the causal
@@ -135,8 +238,7 @@ struct MfmaArgs {
   int nm;
   int tiles;  // 16-row tiles of all matrices
   int G, T;   // 128-column groups; tokens
-  const unsigned char *dig;
-  const float *asc;
+  MixDigits d;
   // causal convolution on matrix 0
   float *conv_state;    // [slot][K][channels]
   const float *conv_w;  // [channels][K]
@@ -196,7 +298,10 @@ __global__ __launch_bounds__(64 * W) void k_mix_mfma(MfmaArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   float *const red = (float *)smem;  // [parity][wave][token][pitch]
   uint64_t *const etab = (uint64_t *)(smem + kMfmaRed);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, kb = lane >> 4;
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, kb = lane >> 4;
+  // in a scalar register, and what follows from it (W 16, GW 4 spills without:
+  // the 16-token S397 out projection 14.5 against 11.7 us)
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   unsigned char *const ring = smem + kMfmaRed + 256 + wave * (NR * Ring::wave);
   const int t0 = blockIdx.y * kDigTile, nt = a.T - t0 < kDigTile ? a.T - t0 : kDigTile;
   const int g0 = wave * GW, tiles = a.tiles, step = gridDim.x;
@@ -245,8 +350,8 @@ __global__ __launch_bounds__(64 * W) void k_mix_mfma(MfmaArgs a) {
   copy(blockIdx.x, 0);
   // lanes of absent tokens read token 0's digits: no more lines
   const unsigned char *const dp =
-      a.dig + (size_t)blockIdx.y * a.G * (kDigPlanes * 1024) + (kb * 16 + (n < nt ? n : 0)) * 16;
-  const float *const ap = a.asc + (size_t)blockIdx.y * a.G * kDigTile + (n < nt ? n : 0);
+      a.d.dig + (size_t)blockIdx.y * a.G * (kDigPlanes * 1024) + (kb * 16 + (n < nt ? n : 0)) * 16;
+  const float *const ap = a.d.asc + (size_t)blockIdx.y * a.G * kDigTile + (n < nt ? n : 0);
   v4i dv[ND][kDigPlanes];
   float av[GW];
   auto digits = [&](int b, int g) {
@@ -264,8 +369,13 @@ __global__ __launch_bounds__(64 * W) void k_mix_mfma(MfmaArgs a) {
 #pragma unroll
       for (int d = 0; d < kDigPlanes; d++) asm volatile("" : "+v"(dv[i][d]));
   }
+  unsigned left = 0;  // groups in which a token has columns outside the digits
 #pragma unroll
-  for (int i = 0; i < GW; i++) asm volatile("" : "+v"(av[i]));
+  for (int i = 0; i < GW; i++) {
+    if (__ballot(__float_as_uint(av[i]) >> 31) != 0) left |= 1u << i;
+    av[i] = fabsf(av[i]);
+    asm volatile("" : "+v"(av[i]));
+  }
   for (int i = 1; i < NR - 1; i++)
     if ((int)blockIdx.x + i * step < tiles) copy(blockIdx.x + i * step, i);
 
@@ -309,7 +419,7 @@ __global__ __launch_bounds__(64 * W) void k_mix_mfma(MfmaArgs a) {
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         const float f = __builtin_fmaf((float)(c[0][e] * 256 + c[1][e]), 65536.0f, (float)(c[2][e] * 256 + c[3][e]));
-        acc[e] = __builtin_fmaf(f, s4[e] * as, acc[e]);
+        acc[e] = FMT == 4 ? __builtin_fmaf(f * as, s4[e], acc[e]) : __builtin_fmaf(f, as, acc[e]);
       }
     };
     // groups past the row add their scale 0
@@ -325,6 +435,19 @@ __global__ __launch_bounds__(64 * W) void k_mix_mfma(MfmaArgs a) {
         if (j + 2 < GW) digits(0, g0 + j + 2);
         group(j + 1, 1, av[j + 1]);
       }
+    }
+#pragma unroll 1
+    for (unsigned u = left; u; u &= u - 1) {
+      const int j = __builtin_ctz(u);
+      int l = lane;
+      asm volatile("" : "+v"(l));  // addresses formed here, not held in registers through the launch
+      const int ln = l & 15, row = 4 * (l >> 4), tok = ln < nt ? ln : 0;
+      add_left_out(a.d.mask + (((size_t)blockIdx.y * a.G + g0 + j) * kDigTile + tok) * 16,
+                   a.d.out + ((size_t)(t0 + tok) * a.G + g0 + j) * 128,
+                   FMT == 4 ? *(const v4f *)(sc + 16 * j + row) : v4f{1.f, 1.f, 1.f, 1.f}, acc, [&](int e, int c) {
+                     const int at = FMT == 4 ? j * 1024 + ((c & 31) >> 1) : (2 * j + (c >> 4 & 1)) * 1024 + (c & 15);
+                     return code_of<FMT>(slot[at + 16 * ((c >> 5) * 16 + row + e)], c);
+                   });
     }
     *(v4f *)(red + ((p % Ring::parities * W + wave) * kDigTile + n) * kMfmaPitch + 4 * kb) = acc;
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -385,7 +508,8 @@ template <int FMT>
 __global__ __launch_bounds__(512) void k_mix_gemm(MfmaArgs a) {
   constexpr int NA = FMT == 4 ? 1 : 2, RT = 4, NTW = 2;
   extern __shared__ __align__(16) unsigned char smem[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, kb = lane >> 4;
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, kb = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave & 1, wn = wave >> 1;
   const int ttiles = (a.T + kDigTile - 1) / kDigTile, tb = (ttiles + kGemmTiles - 1) / kGemmTiles;
   const int rb = blockIdx.x / tb, tile0 = (blockIdx.x % tb) * kGemmTiles;
@@ -413,12 +537,12 @@ __global__ __launch_bounds__(512) void k_mix_gemm(MfmaArgs a) {
 #pragma unroll
     for (int j = 0; j < kGemmTiles; j++) {  // wave w copies plane w of every tile
       const int tt = tile0 + j < ttiles ? tile0 + j : ttiles - 1;
-      dma_b128(a.dig + (((size_t)tt * a.G + g) * kDigPlanes + wave) * 1024 + 16 * lane,
+      dma_b128(a.d.dig + (((size_t)tt * a.G + g) * kDigPlanes + wave) * 1024 + 16 * lane,
                lds_addr(buf + (j * kDigPlanes + wave) * 1024));
     }
     if (wave < NTW) {
       const int j = 4 * wave + kb, tt = tile0 + j < ttiles ? tile0 + j : ttiles - 1;
-      dma_b32(a.asc + ((size_t)tt * a.G + g) * kDigTile + n, lds_addr(buf + kGemmScales + wave * 256));
+      dma_b32(a.d.asc + ((size_t)tt * a.G + g) * kDigTile + n, lds_addr(buf + kGemmScales + wave * 256));
     }
     if (FMT == 4 && wave >= 6) {
       const int row = row0 + 64 * (wave - 6) + lane;
@@ -431,6 +555,7 @@ __global__ __launch_bounds__(512) void k_mix_gemm(MfmaArgs a) {
   for (int r = 0; r < RT; r++)
 #pragma unroll
     for (int j = 0; j < NTW; j++) acc[r][j] = v4f{0.f, 0.f, 0.f, 0.f};
+  unsigned long long left[NTW] = {};  // groups in which a token has columns outside the digits (G <= kMfmaMaxGroups)
   copy(0, 0);
   weights(0);
   for (int g = 0; g < a.G; g++) {
@@ -469,7 +594,8 @@ __global__ __launch_bounds__(512) void k_mix_gemm(MfmaArgs a) {
       v4i d[kDigPlanes];
 #pragma unroll
       for (int p = 0; p < kDigPlanes; p++) d[p] = *(const v4i *)(buf + (tl * kDigPlanes + p) * 1024 + 16 * lane);
-      const float as = *(const float *)(buf + kGemmScales + (tl * kDigTile + n) * 4);
+      const float sas = *(const float *)(buf + kGemmScales + (tl * kDigTile + n) * 4), as = fabsf(sas);
+      if (__ballot(__float_as_uint(sas) >> 31) != 0) left[j] |= 1ull << g;
 #pragma unroll
       for (int r = 0; r < RT; r++) {
         v4i c[4];
@@ -480,8 +606,30 @@ __global__ __launch_bounds__(512) void k_mix_gemm(MfmaArgs a) {
 #pragma unroll
         for (int e = 0; e < 4; e++) {
           const float f = __builtin_fmaf((float)(c[0][e] * 256 + c[1][e]), 65536.0f, (float)(c[2][e] * 256 + c[3][e]));
-          acc[r][j][e] = __builtin_fmaf(f, s4[r][e] * as, acc[r][j][e]);
+          acc[r][j][e] = FMT == 4 ? __builtin_fmaf(f * as, s4[r][e], acc[r][j][e]) : __builtin_fmaf(f, as, acc[r][j][e]);
         }
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < NTW; j++) {
+    const int tl = tile0 + wn * NTW + j, tt = tl < ttiles ? tl : ttiles - 1, t = tt * kDigTile + n;
+#pragma unroll 1
+    for (unsigned long long u = left[j]; u; u &= u - 1) {
+      const int g = __builtin_ctzll(u);
+#pragma unroll
+      for (int r = 0; r < RT; r++) {
+        const unsigned char *q[4];
+        v4f s4;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const int row = row0 + 64 * wm + 16 * r + 4 * kb + e, rc = row < rlast ? row : rlast;
+          q[e] = pm.q + (size_t)rc * pm.rb + (size_t)g * (FMT == 4 ? 64 : 128);
+          s4[e] = FMT == 4 ? pm.s[(size_t)rc * pm.ng + g] : 1.0f;
+        }
+        add_left_out(a.d.mask + (((size_t)tt * a.G + g) * kDigTile + n) * 16,
+                     a.d.out + ((size_t)(t < a.T ? t : 0) * a.G + g) * 128, s4, acc[r][j],
+                     [&](int e, int c) { return code_of<FMT>(q[e][FMT == 4 ? c >> 1 : c], c); });
       }
     }
   }
