@@ -34,8 +34,8 @@ using namespace sw;
 // row: the block writes a chunk of squares to LDS, one wave adds them in
 // order (serial_sum_nonneg), the next chunk follows.
 // Aligned rows of n <= 4096: one read of x as float4, kept in registers with
-// the weights while the sum is formed.  512 rows of 2,048: 18.4 -> 11 us (7.5 us
-// before without its sum).
+// the weights while the sum is formed.  512 rows of 2,048: 17.0 -> 10.2 us, 12.6
+// of bf16 values.
 constexpr int kNormChunk = 4096;
 __global__ __launch_bounds__(256) static void k_rmsnorm_zero4(float *y, const float *x, const float *w, int n,
                                                               float eps) {

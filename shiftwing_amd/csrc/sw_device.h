@@ -251,10 +251,9 @@ __device__ __forceinline__ float serial_sum_lds(const float *p, int m, float s =
 #pragma unroll
     for (int k = 0; k < 8; k++) b[k] = ((const float4 *)(p + i + 32))[k];
     add32(s, a);
-    if (i + 64 < m) {
+    const float *const nx = p + (i + 64 < m ? i + 64 : i);
 #pragma unroll
-      for (int k = 0; k < 8; k++) a[k] = ((const float4 *)(p + i + 64))[k];
-    }
+    for (int k = 0; k < 8; k++) a[k] = ((const float4 *)nx)[k];
     add32(s, b);
   }
   return s;
@@ -271,18 +270,38 @@ __device__ __forceinline__ float serial_sum_lds(const float *p, int m, float s =
 // with a second tie, a term of 2^23 u or more, or a sum that reaches 2^24 u
 // ends the run: its terms are added as written and the rest go on from there.
 // A sum that grows from its first terms has one binade step and about one tie
-// per doubling; the first 64 terms, where every few end a run, are added one by
-// one, and so are sums too small or large for exact scaling.  A run is about 750 cycles of dependent code: 2,048 squares in 11 us by
-// one lane's dependent adds, 5 us this way.
+// per doubling if the terms have full 24-bit mantissas; the first 64 terms,
+// where every few end a run, are added one by one, and so are sums too small or
+// large for exact scaling.  A run is about 750 cycles of dependent code, as
+// long as 57 dependent adds.  Squares of shorter mantissas (bf16 activations,
+// integers) tie far more often, growing rows change binade: a step with more
+// than kSerialTies tied lanes ahead of it, or kSerialRuns ended runs behind it,
+// adds its rest one by one, and after kSerialBad steps that left more than half
+// of themselves so, the row does.  A norm of 2,048 / 4,096 values by one lane's
+// adds alone 12.1 / 22.7 us; this way 6.6 / 11.0 of full mantissas, 9.6 / 16.9 of
+// bf16 values (62 / 70 without the bound), 9.4 / 16.2 of nothing but ties (144 / 290).
 constexpr int kSerialStep = 512;
+constexpr int kSerialRuns = 4, kSerialTies = 6, kSerialBad = 2;
 __device__ __forceinline__ float lane_value(float v, int l) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
 }
 __device__ __forceinline__ float serial_sum_nonneg(const float *p, int m, float s) {
   const int lane = threadIdx.x & 63;
-  const bool fresh = s == 0.0f;
-  if (fresh) s = serial_sum_lds(p, 64);
-  for (int c = 0; c < m; c += kSerialStep) {
+  const int mp = (m + 63) & ~63;
+  int bad = 0;
+  // terms from `at` on that are added one by one: the first 64, or all of a
+  // step and less (as long either way)
+  int at = 0, todo = m <= kSerialStep ? mp : s == 0.0f ? 64 : 0;
+  while (at < m) {
+    if (todo > 0) {
+      s = serial_sum_lds(p + at, todo, s);
+      at += todo;
+      todo = 0;
+      continue;
+    }
+    const int c = at & ~(kSerialStep - 1);
+    int l0 = (at - c) >> 3;  // lanes below l0 are in s
+    at = c + kSerialStep;
     float v[8];
     *(float4 *)v = ((const float4 *)(p + c))[2 * lane];
     *(float4 *)(v + 4) = ((const float4 *)(p + c))[2 * lane + 1];
@@ -291,8 +310,12 @@ __device__ __forceinline__ float serial_sum_nonneg(const float *p, int m, float 
 #pragma unroll
     for (int j = 0; j < 8; j++) some |= !(v[j] == 0.0f);
     if (__ballot(some) == 0) continue;
-    int l0 = fresh && c == 0 ? 8 : 0;  // lanes below l0 are in s
-    while (l0 < 64) {
+    bool plain = false;
+    for (int runs = 0; l0 < 64 && !plain; runs++) {
+      if (runs == kSerialRuns) {
+        plain = true;
+        break;
+      }
       const unsigned sb = __builtin_amdgcn_readfirstlane((int)__float_as_uint(s));
       const int e = (int)(sb >> 23);
       int f = l0;
@@ -310,6 +333,10 @@ __device__ __forceinline__ float serial_sum_nonneg(const float *p, int m, float 
         }
         int sum = 0, ties = 0, at_tie = 0;
         const unsigned long long tied = __ballot(on && tie && !big);
+        if (__builtin_popcountll(tied) > kSerialTies) {
+          plain = true;
+          break;
+        }
         if (tied) {  // ties rounded down here
 #pragma unroll
           for (int j = 0; j < 8; j++) {
@@ -342,6 +369,7 @@ __device__ __forceinline__ float serial_sum_nonneg(const float *p, int m, float 
         const unsigned long long ends = __ballot(on && (big || ties > 0 || S + inc >= (1 << 24)));
         if (ends == 0) {
           s = (float)(S + __builtin_amdgcn_readlane(inc, 63)) * u;
+          l0 = 64;
           break;
         }
         f = __builtin_ctzll(ends);
@@ -350,6 +378,14 @@ __device__ __forceinline__ float serial_sum_nonneg(const float *p, int m, float 
 #pragma unroll
       for (int j = 0; j < 8; j++) s = __fadd_rn(s, lane_value(v[j], f));
       l0 = f + 1;
+    }
+    if (plain) {
+      for (; l0 & 7; l0++)
+#pragma unroll
+        for (int j = 0; j < 8; j++) s = __fadd_rn(s, lane_value(v[j], l0));
+      bad += l0 < 32;
+      at = c + 8 * l0;
+      todo = (bad < kSerialBad ? c + kSerialStep : mp) - at;
     }
   }
   return s;
