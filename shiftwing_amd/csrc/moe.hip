@@ -1200,12 +1200,18 @@ __device__ void topk_check_token(Work &w, int t, unsigned long long *stats) {
 // with coalesced loads into LDS, then one lane runs the serial sum over LDS,
 // s = rn(s + p_i), and the fused tail.  Same result as exact_chain.
 // Blocks walk the list of uncertain tokens (few: most launches find none).
-// grid (kUncertainChains, min(T, kUncertainSlots)), 64 threads, dynamic LDS
-// 4*H bytes: a token's set holds little more than K experts, and 1,999 tokens
-// leave some 150 uncertain (64 x 128 blocks walked them in two rounds, 110 us
-// at S397, 26 us for the 512 tokens of an S35 chunk; 16 x 512 90 and 17 us).
+// grid (uncertain_chains(K), min(T, kUncertainBlocks / chains)), 64 threads,
+// dynamic LDS 4*H bytes.  A token's set holds little more than K experts, and a
+// chain that finds no block waits a whole round of 26 us (4,096 products); blocks
+// without a chain take the place of a token's, where many are uncertain.  Routing
+// at 16 / 24 / 32 / 64 chains: K 8 353 / 355 / 378 / 382 us (1,999 S397 tokens) and
+// 69 / 69 / 71 / 76 (512 S35), K 16 77 / 62 / 62 / 63 (32 S397 tokens) and 624 / 605 /
+// 649 / 674 (1,999), K 20 70 / 53 / 54 / 54 (8) and 870 / 812 / 857 / 870, K 24 85 / 67 /
+// 68 / 73 (32) and 137 / 128 / 125 / 123 (64), K 32 78 / 78 / 60 / 60 (8) and 159 / 151 /
+// 145 / 134 (64).
 // ---------------------------------------------------------------------------
-constexpr int kUncertainChains = 16, kUncertainSlots = 512;
+constexpr int kUncertainBlocks = 8192;
+static int uncertain_chains(int K) { return K > 24 ? 64 : (K + 15) & ~7; }
 __global__ __launch_bounds__(64) void k_exact_logits(Work w, const float *x, const float *router,
                                                      unsigned long long *stats) {
   extern __shared__ float prod[];
@@ -3399,8 +3405,8 @@ static int route_launch(ColiCuda *ctx, ColiMoeLayer *L, Work &w, const float *x)
       k_certify<<<w.T, 512, 0, st>>>(w, L->router_mode, L->stats);
   }
   if (set_lds((const void *)k_exact_logits, (size_t)w.H * 4)) return -1;
-  k_exact_logits<<<dim3(kUncertainChains, w.T < kUncertainSlots ? w.T : kUncertainSlots), 64, (size_t)w.H * 4, st>>>(
-      w, x, L->router, L->stats);
+  const int chains = uncertain_chains(w.K), uslots = kUncertainBlocks / chains;
+  k_exact_logits<<<dim3(chains, w.T < uslots ? w.T : uslots), 64, (size_t)w.H * 4, st>>>(w, x, L->router, L->stats);
   const int e4 = (w.E + 3) & ~3;
   const size_t full_lds = (size_t)4 * (w.H > 2 * e4 ? w.H : 2 * e4);
   if (set_lds((const void *)k_exact_full, full_lds)) return -1;
