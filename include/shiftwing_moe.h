@@ -515,10 +515,11 @@ int coli_cuda_moe_decode_times(ColiCuda *ctx, double ms[3],
  * not take fall back to 2); 2 the three per-layer decode kernels; 0 the
  * many-token kernels.  Same results to the stated tolerance (for tests). */
 int coli_cuda_moe_set_decode_kernels(ColiCuda *ctx, int mode);
-/* Many-token steps: tokens per expert work item.  0 (default) picks 16 (each
- * expert's tiles read once per 16 tokens) when an item's activation digits
- * fit the LDS, else 8; 8 or 16 force one.  Same indices; outputs to the
- * stated tolerance (for tests and measurement). */
+/* Many-token steps: tokens per expert work item.  0 (default) picks 64 where
+ * experts hold many tokens on average and the items fill the device, else 16
+ * (each expert's tiles read once per 16 tokens) when an item's activation
+ * digits fit the LDS, else 8; 8, 16 or 64 force one.  Same indices; outputs to
+ * the stated tolerance (for tests and measurement). */
 int coli_cuda_moe_set_item_tokens(ColiCuda *ctx, int tokens);
 /* Stage stamps of the persistent decode kernel (measurement): while set,
  * every call writes the device wall clock (100 MHz) into the caller's device

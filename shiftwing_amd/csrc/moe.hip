@@ -250,7 +250,7 @@ constexpr int kShSplit = 4, kShSplitTokens = SW_SH_SPLIT_TOKENS;
 // ---------------------------------------------------------------------------
 struct Work {
   int T, H, E, K, I, Ish, ngh, ngi, Hp, Ip;
-  int itok;  // tokens per bucketing item: 8 (one MFMA column set) or kWideTokens
+  int itok;  // tokens per bucketing item: 8 (one MFMA column set), kWideTokens or kTallTokens
   // 1 when the step returns no routes: a certified set of K experts is taken
   // in the order of its bounds when they cannot settle it (the set is exact
   // either way, the weights come from the fp64 logits within tolerance; only
@@ -3421,17 +3421,32 @@ static int route_launch(ColiCuda *ctx, ColiMoeLayer *L, Work &w, const float *x)
 // no block barrier, and are faster at every step size measured, however few
 // tokens an expert holds (S397: 834 against 686 tok/s at 8 tokens a step,
 // 1763 against 1388 at 32).  The context's setting
-// (coli_cuda_moe_set_item_tokens) can force either.  Tall items from
-// kTallMinTokens tokens an expert on average, against wide ones: S397 at 10 / 16 /
-// 20 / 39 tokens an expert 992 / 1122 / 1289 / 1978 against 920 / 1180 / 1489 / 2389
-// us a step, S35 at 16 / 20 / 32 / 47 270 / 304 / 396 / 463 against 255 / 310 / 422 /
-// 517.
-constexpr int kTallMinTokens = 18;
+// (coli_cuda_moe_set_item_tokens) can force any.
+// Tall items pay where experts hold many tokens and the items fill the device:
+// with n tokens an expert on average and W gate/up workgroups (items times
+// 128-value groups of I, two of them resident a compute unit) they win from about
+// n = 30 at W = 1,024 and n = 18 at 4,096, n^2 W constant between.  Step time tall /
+// wide, uniform and Zipf routing (skew leaves most items few tokens):
+//   S397 (W 4,096)                n 18 .90 .92, 24 .83 .89, 40 .78 .81
+//   S35 (1,024)                   n 18 .98 1.10, 24 .97 1.04, 32 .94 1.02, 40 .87 1.00
+//   H 4,096, 128 of 1,024 (1,024) n 18 .99 1.06, 24 .93 1.04, 32 .87 .96
+//   H 3,072, 128 of 768 (768)     n 18 1.05 1.11, 32 .93 .98, 40 .89 .95
+//   H 4,096, 32 of 2,048 (512)    n 32 .92 1.05, 40 .90 .98, 64 .89 .88
+//   H 2,048, 64 of 768 (384)      n 18 1.02 1.13, 40 1.01 1.04, 64 1.06 1.06
+//   H 1,024, 64 of 512 (256, 512) n 40 1.07 1.13, 100 1.02 1.04: rows of 8 groups
+// and 16 experts of 512 at n 18 / 54 / 108 (64 to 128) 1.12 / 1.20 / 1.12.
+static bool tall_pays(const ColiCuda *ctx, const ColiMoeLayer *L, int T) {
+  const long long routes = (long long)T * L->sh.topk, E = L->sh.experts;
+  const int cus = ctx->sm_count > 0 ? ctx->sm_count : 256;
+  const long long W = E * ((routes + kTallTokens * E - 1) / (kTallTokens * E)) * L->ngi;
+  return L->ngh >= 16 && routes >= 18 * E && W >= 2 * cus &&
+         (double)routes / E * ((double)routes / E) * W >= 900.0 * 4 * cus;
+}
 static int item_tokens(const ColiCuda *ctx, const ColiMoeLayer *L, int T) {
   const int mode = ctx->moe_item_tokens;
   const bool fits = wide_lds_bytes(wide_stage_groups(L->ngh, kWideGuBatch)) <= 160 * 1024 &&
                     wide_lds_bytes(wide_stage_groups(L->ngi, kWideDnBatch)) <= 160 * 1024;
-  if (mode == 0 && (long long)T * L->sh.topk >= (long long)kTallMinTokens * L->sh.experts) return kTallTokens;
+  if (mode == kTallTokens || (mode == 0 && tall_pays(ctx, L, T))) return kTallTokens;
   return fits && mode != kMaxTokensPerItem ? kWideTokens : kMaxTokensPerItem;
 }
 
@@ -3597,7 +3612,7 @@ extern "C" int coli_cuda_moe_forward(ColiCuda *ctx, ColiMoeLayer *L, float *y, c
   }
   mark(ctx, 4);
   prof_mark(ctx, kStageRoutedHidden);
-  if (!wide_items) k_prep_hidden<<<T + T * w.K, 256, 0, st>>>(w, L->sh_gs, L->sh_us);  // else in k_gateup_wide
+  if (!wide_items) k_prep_hidden<<<T + T * w.K, 256, 0, st>>>(w, L->sh_gs, L->sh_us);  // else in the gate/up kernel, or before it
   mark(ctx, 5);
   int sh_chunks = (T + kSharedTokens - 1) / kSharedTokens;
   const int dn_blocks_x = (w.H / kTileRows + 4 * kDnRowTiles - 1) / (4 * kDnRowTiles);
@@ -3744,9 +3759,9 @@ extern "C" int coli_cuda_moe_decode_times(ColiCuda *ctx, double ms[3], unsigned 
 }
 
 extern "C" int coli_cuda_moe_set_item_tokens(ColiCuda *ctx, int tokens) {
-  if (!ctx || (tokens != 0 && tokens != kMaxTokensPerItem && tokens != kWideTokens))
-    return fail_arg("coli_cuda_moe_set_item_tokens: %d (0 automatic, %d or %d)", tokens, kMaxTokensPerItem,
-                    kWideTokens);
+  if (!ctx || (tokens != 0 && tokens != kMaxTokensPerItem && tokens != kWideTokens && tokens != kTallTokens))
+    return fail_arg("coli_cuda_moe_set_item_tokens: %d (0 automatic, %d, %d or %d)", tokens, kMaxTokensPerItem,
+                    kWideTokens, kTallTokens);
   ctx->moe_item_tokens = tokens;
   return 0;
 }

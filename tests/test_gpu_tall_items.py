@@ -1,5 +1,5 @@
-"""Steps whose experts hold many tokens (items of 64) against the same step in
-items of 16: the same arithmetic per (row, token) in the same order, so equal
+"""Steps in items of 64 tokens (forced: the automatic choice is another test's)
+against the same step in items of 16: the same arithmetic per (row, token) in the same order, so equal
 bits; and against the oracle.  Shapes at the edges: row tiles of I and H that
 do not fill a workgroup, partial 128-column groups, one group, experts with 0,
 1, 16, 17, 64, 65 and more tokens, int3, int4 and int2."""
@@ -40,7 +40,7 @@ def test_tall_items_equal_wide_items(be, oracle, H, E, K, I, Ish, fmt, T):
     x = np.random.default_rng(92).standard_normal((T, H)).astype(np.float32)
     print(f"[tall items] H={H} E={E} K={K} I={I} fmt={fmt} T={T}", flush=True)
     y0, i0, w0 = _forward(be, L, x, 16)
-    y1, i1, w1 = _forward(be, L, x, 0)
+    y1, i1, w1 = _forward(be, L, x, 64)
     assert np.array_equal(i0, i1) and np.array_equal(w0, w1)
     assert np.array_equal(y0.view(np.uint32), y1.view(np.uint32))
     hl = oracle.host_layer(91, 0, H, E, K, I, Ish, fmt)
@@ -67,7 +67,7 @@ def test_tall_items_uneven_experts(be):
     x[:, :E] = 0.0
     x[np.arange(which.size), which] = 8.0
     y0, i0, _ = _forward(be, L, x, 16)
-    y1, i1, _ = _forward(be, L, x, 0)
+    y1, i1, _ = _forward(be, L, x, 64)
     assert np.array_equal(i1[:, 0], which) and np.array_equal(i0, i1)
     assert np.array_equal(y0.view(np.uint32), y1.view(np.uint32))
     L.close()
