@@ -1505,8 +1505,13 @@ int gqa_run(ColiCuda *ctx, const GqaCall &c) {
     }
     sp.first[R] = wgs;
   } else {
+    // one row, or a prompt chunk of few: one workgroup a compute unit until
+    // each has three blocks a wave, since the merge grows with the splits.  One
+    // row at 8,193 / 12,289 / 16,385 / 24,577 / 65,537 keys, one against two: S397
+    // 46.1 / 48.0 / 52.2 / 58.1 / 90.5 against 48.8 / 50.4 / 53.5 / 57.5 / 88.0 us, S35
+    // 38.5 / 40.2 / 44.6 / 50.4 / 79.0 against 40.1 / 41.7 / 44.6 / 47.5 / 75.4
     const int nb = c.max_pos / 16 + 1;
-    int S = target / (c.nkv * R);
+    int S = ((long long)nb * c.nkv * R < 6LL * target ? target / 2 : target) / (c.nkv * R);
     const int smax = (nb + kAttnWaves - 1) / kAttnWaves;
     S = S > smax ? smax : S;
     S = S > kMaxSplits ? kMaxSplits : S;
