@@ -377,7 +377,9 @@ extern "C" int coli_cuda_q3_gemv_f16(ColiCuda *ctx, float *y, const unsigned sho
 // ---------------------------------------------------------------------------
 // grouped routed experts over caller pointer tables (backend_cuda.h:87-118).
 // The tables and the route weights travel as kernel arguments (64 routes, 3.4
-// KB), so a call is two launches and no copy: the hidden vectors of every
+// KB), so a call is two launches and no copy (route weights in memory that the
+// device may still write, page-locked or its own, are copied in stream order):
+// the hidden vectors of every
 // route, then a wave per (token, output row) that takes the token's routes in
 // turn and adds them in route order.  Latency-bound: four S35 tokens (37 MB)
 // took two launches of each stage at 16 routes a table, a weight upload and a
@@ -411,11 +413,11 @@ __global__ static void k_grouped_hidden(float *h, const XT *x, HiddenTable t, in
   if (lane == 0) h[(size_t)r * I + row] = silu_ref(g) * u;
 }
 
-// y[b, row] = sum_j w[b*K+j] * (down_{b*K+j} . h[b*K+j])[row] (j ascending);
-// grid (ceil(H/4), batch)
-template <int BITS>
-__global__ static void k_grouped_down(float *y, const float *h, DownTable t, int K, int H, int I, int gs, int rb,
-                                      int groups) {
+// y[b, row] = sum_j w[b*K+j] * (down_{b*K+j} . h[b*K+j])[row] (j ascending), w
+// from `dw` (DW) or the table; grid (ceil(H/4), batch)
+template <int BITS, bool DW>
+__global__ static void k_grouped_down(float *y, const float *h, DownTable t, const float *dw, int K, int H, int I, int gs,
+                                      int rb, int groups) {
   int lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6), b = blockIdx.y;
   if (row >= H) return;
   float total = 0.0f;
@@ -423,9 +425,21 @@ __global__ static void k_grouped_down(float *y, const float *h, DownTable t, int
     const int r = b * K + j;
     const float v = wave_sum_dpp(lane_dot_qx<BITS, float>(t.dq[r] + (size_t)row * rb, t.ds[r] + (size_t)row * groups,
                                                           h + (size_t)r * I, I, gs, lane));
-    total += t.w[r] * v;
+    total += (DW ? dw[r] : t.w[r]) * v;
   }
   if (lane == 0) y[(size_t)b * H + row] = total;
+}
+
+// Memory that queued work may still write before the stream reaches a call:
+// page-locked host memory and device memory.  Pageable memory is the host's alone.
+static bool stream_ordered_memory(const void *p) {
+  hipPointerAttribute_t a;
+  memset(&a, 0, sizeof(a));
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return a.type != hipMemoryTypeUnregistered;
 }
 
 template <int BITS, typename XT>
@@ -437,7 +451,12 @@ static int grouped_mlp(ColiCuda *ctx, const char *name, float *y, const XT *x,
                        int hgroups, int drb, int dgroups) {
   const int routes = batch * K;
   if (ensure_scratch(ctx, kScrHidden, (size_t)routes * I * sizeof(float), "grouped hidden allocation")) return -1;
-  float *h = (float *)ctx->scratch[kScrHidden];
+  float *h = (float *)ctx->scratch[kScrHidden], *dw = nullptr;
+  const bool ordered = stream_ordered_memory(route_weight);
+  if (ordered) {
+    if (ensure_scratch(ctx, kScrWeight, (size_t)routes * sizeof(float), "grouped weight allocation")) return -1;
+    dw = (float *)ctx->scratch[kScrWeight];
+  }
   prof_open(ctx);
   HiddenTable ht;
   DownTable dt;
@@ -452,12 +471,21 @@ static int grouped_mlp(ColiCuda *ctx, const char *name, float *y, const XT *x,
     ht.us[i] = up_s[i];
     dt.dq[i] = down_q[i];
     dt.ds[i] = down_s[i];
-    dt.w[i] = route_weight[i];  // host values (c/backend_cuda.cu:1568)
+    if (!ordered) dt.w[i] = route_weight[i];  // host values (c/backend_cuda.cu:1568)
+  }
+  if (ordered) {
+    const hipError_t e =
+        hipMemcpyAsync(dw, route_weight, (size_t)routes * sizeof(float), hipMemcpyHostToDevice, ctx->stream);
+    if (e != hipSuccess) return fail_hip("grouped route weight upload", e);
   }
   prof_mark(ctx, kStageSetup);
   k_grouped_hidden<BITS, XT><<<dim3((I + 3) / 4, routes), 256, 0, ctx->stream>>>(h, x, ht, K, I, H, gs, hrb, hgroups);
   prof_mark(ctx, kStageRoutedHidden);
-  k_grouped_down<BITS><<<dim3((H + 3) / 4, batch), 256, 0, ctx->stream>>>(y, h, dt, K, H, I, gs, drb, dgroups);
+  const dim3 grid((H + 3) / 4, batch);
+  if (ordered)
+    k_grouped_down<BITS, true><<<grid, 256, 0, ctx->stream>>>(y, h, dt, dw, K, H, I, gs, drb, dgroups);
+  else
+    k_grouped_down<BITS, false><<<grid, 256, 0, ctx->stream>>>(y, h, dt, dw, K, H, I, gs, drb, dgroups);
   prof_mark(ctx, kStageRoutedDown);
   int st = launch_status(name);
   if (!st) prof_mark(ctx, kStageReduce);

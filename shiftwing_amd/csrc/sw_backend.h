@@ -28,8 +28,9 @@
 namespace sw {
 
 enum Scratch {
-  kScrSetup = 0,   // reference grouped calls: route weights on the device
+  kScrSetup = 0,   // layer setup: stored experts while they are widened or synthesized
   kScrHidden,      // reference grouped calls: routed hidden activations
+  kScrWeight,      // reference grouped calls: route weights of page-locked memory
   kScrGate,        // reference shared-expert calls: hidden vectors, gate logits
   kScrUp,
   kScrXPrep,       // many-token step: activation digits, routes, buckets
