@@ -430,18 +430,6 @@ __global__ static void k_grouped_down(float *y, const float *h, DownTable t, con
   if (lane == 0) y[(size_t)b * H + row] = total;
 }
 
-// Memory that queued work may still write before the stream reaches a call:
-// page-locked host memory and device memory.  Pageable memory is the host's alone.
-static bool stream_ordered_memory(const void *p) {
-  hipPointerAttribute_t a;
-  memset(&a, 0, sizeof(a));
-  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
-    (void)hipGetLastError();
-    return false;
-  }
-  return a.type != hipMemoryTypeUnregistered;
-}
-
 template <int BITS, typename XT>
 static int grouped_mlp(ColiCuda *ctx, const char *name, float *y, const XT *x,
                        const unsigned char *const *gate_q, const float *const *gate_s,

@@ -91,6 +91,24 @@ int ensure_scratch(ColiCuda *ctx, Scratch which, size_t bytes, const char *where
   return 0;
 }
 
+bool stream_ordered_memory(const void *p) {
+  hipPointerAttribute_t a;
+  memset(&a, 0, sizeof(a));
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return a.type != hipMemoryTypeUnregistered;
+}
+
+char *host_block(ColiCuda *ctx) {
+  if (!ctx->host_block && hipHostMalloc((void **)&ctx->host_block, 2 * kHostBlock, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    ctx->host_block = nullptr;
+  }
+  return ctx->host_block;
+}
+
 // ---- block cache ------------------------------------------------------------
 
 static void cache_trim(ColiCuda *ctx) {
@@ -314,6 +332,7 @@ extern "C" void coli_cuda_destroy(ColiCuda *ctx) {
   cache_trim(ctx);  // blocks the caller still holds are the caller's
   for (void *p : ctx->scratch)
     if (p) (void)hipFree(p);
+  if (ctx->host_block) (void)hipHostFree(ctx->host_block);
   stack_release(ctx);
   for (hipEvent_t ev : ctx->prof.events) (void)hipEventDestroy(ev);
   if (ctx->prof.stamps) (void)hipFree(ctx->prof.stamps);

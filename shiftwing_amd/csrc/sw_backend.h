@@ -93,6 +93,7 @@ struct ColiCuda {
   sw::BlockCache cache;
   sw::StageProfiler prof;
   void *scratch[sw::kScrCount] = {};
+  char *host_block = nullptr;  // page-locked staging of small host arrays
   size_t scratch_cap[sw::kScrCount] = {};
   // stream timer and MoE stage timing
   hipEvent_t timer_event[2] = {};
@@ -138,6 +139,16 @@ int fail_arg(const char *fmt, ...);
 int launch_status(const char *where);
 // Grow-only scratch owned by the context (released by coli_cuda_destroy).
 int ensure_scratch(ColiCuda *ctx, Scratch which, size_t bytes, const char *where);
+
+// Memory that queued work may still write before the stream reaches a call:
+// page-locked host memory and device memory.  Pageable memory is the host's alone.
+bool stream_ordered_memory(const void *p);
+// The context's page-locked block, kHostBlock bytes for inputs and as many
+// behind them for outputs, allocated at the first call (nullptr where it cannot
+// be had), for the host arrays of calls that wait for the stream before they
+// return.
+constexpr size_t kHostBlock = 512 * 1024;
+char *host_block(ColiCuda *ctx);
 
 // Stage profiler (no-ops unless CUDA_PROFILE_STAGES is set at create).
 void prof_open(ColiCuda *ctx);                 // a MoE transaction starts here
