@@ -44,7 +44,7 @@ constexpr int kDigBulk = 8;    // values a range needs to stay in the digits
 // What k_mix_digits leaves behind of `tokens` rows of `cols`: the digits, the
 // group scales [tile][group][16 tokens] (sign set: the token has columns
 // outside the digits), the bits of those columns [tile][group][16 tokens][128]
-// and their values [token][cols] (only those are written).
+// (only of such tokens) and their values [token][cols] (only those).
 struct MixDigits {
   unsigned char *dig;
   float *asc;
@@ -119,46 +119,54 @@ __global__ __launch_bounds__(64) void k_mix_digits(DigitArgs a) {
 #pragma unroll
     for (int e = 0; e < 8; e++) v[e] *= r;
   }
-  // magnitudes as integers; infinities and NaNs leave the digits at once
-  unsigned b[8], left = 0;
-#pragma unroll
-  for (int e = 0; e < 8; e++) {
-    b[e] = __float_as_uint(v[e]) & 0x7fffffffu;
-    left |= b[e] >= 0x7f800000u ? 1u << e : 0;
-  }
-  unsigned mb;  // the largest in the digits
+  // A column that leaves: its value is stored and is 0 in the digits.  Each
+  // turn takes one out of one token's digits at least, or is the last; the
+  // first is the last for nearly every group.
+  unsigned left = 0, mb;  // mb: the largest magnitude in the digits, as an integer
   int k;
   float scale;
-  for (;;) {  // each turn takes a value out of one token's digits, or is the last
+#pragma unroll 1
+  for (;;) {
     mb = 0;
 #pragma unroll
-    for (int e = 0; e < 8; e++) mb = !(left >> e & 1) && b[e] > mb ? b[e] : mb;
+    for (int e = 0; e < 8; e++) {
+      const unsigned b = __float_as_uint(v[e]) & 0x7fffffffu;
+      mb = b > mb ? b : mb;
+    }
     mb = row_max_u32(mb);
-    const int E = (int)(mb >> 23), k0 = 29 + 127 - E;
-    k = k0 < 120 ? k0 : 120;
+    // below 2^-91 the scale would leave the normal range: all of it goes out;
+    // infinities and NaNs (which order above them) go first
+    const int E = (int)(mb >> 23);
+    const bool bad = E == 255, tiny = E < 36;
+    k = tiny ? 120 : 29 + 127 - E;
     scale = __uint_as_float((unsigned)(k + 127) << 23);
-    // below 2^-91 the scale would leave the normal range: all of it goes out
-    const bool tiny = k0 > 120;
-    const unsigned lo = tiny ? 1 : (unsigned)(E - 5) << 23;
-    unsigned big = 0;
+    const unsigned lo = bad ? 0x7f800000u : tiny ? 1 : (unsigned)(E - 5) << 23;
+    int cnt = 0;
 #pragma unroll
-    for (int e = 0; e < 8; e++) big |= !(left >> e & 1) && b[e] >= lo ? 1u << e : 0;
-    bool drop = mb != 0 && (row_sum_i32(__builtin_popcount(big)) < kDigBulk || tiny);
+    for (int e = 0; e < 8; e++) cnt += (__float_as_uint(v[e]) & 0x7fffffffu) >= lo;
+    bool drop = mb != 0 && (row_sum_i32(cnt) < kDigBulk || bad || tiny);
     if (__ballot(drop) == 0) break;
-    bool lossy = false;
+    bool lossy = bad || tiny;
 #pragma unroll
     for (int e = 0; e < 8; e++) {
       const float r = v[e] * scale;
-      lossy |= !(left >> e & 1) && r != __builtin_rintf(r);
+      lossy |= r != __builtin_rintf(r);
     }
-    drop = drop && (tiny || (__ballot(lossy) >> (lane & 48) & 0xffff) != 0);
+    drop = drop && (__ballot(lossy) >> (lane & 48) & 0xffff) != 0;
     if (__ballot(drop) == 0) break;
-    if (drop) left |= big;
+#pragma unroll
+    for (int e = 0; e < 8; e++)
+      if (drop && (__float_as_uint(v[e]) & 0x7fffffffu) >= lo) {
+        if (t < a.T) a.d.out[(size_t)t * a.cols + col + e] = v[e];
+        v[e] = 0.0f;
+        left |= 1u << e;
+      }
   }
+  if (t >= a.T) left = 0;  // an absent token of the tile
   unsigned d[4][2] = {};
 #pragma unroll
   for (int e = 0; e < 8; e++) {
-    int q = left >> e & 1 ? 0 : (int)__builtin_rintf(v[e] * scale);
+    int q = (int)__builtin_rintf(v[e] * scale);
     const int w = ROWS8 ? e >> 2 : e & 1, sh = 8 * (ROWS8 ? e & 3 : e >> 1);
 #pragma unroll
     for (int p = 3; p > 0; p--) {
@@ -176,15 +184,9 @@ __global__ __launch_bounds__(64) void k_mix_digits(DigitArgs a) {
       const int half = ROWS8 ? (i & 3) >> 1 : w, dw = ROWS8 ? 2 * (i & 1) + w : i & 3;
       out[(2 * p + half) * 256 + dw] = d[p][w];
     }
-  if (t >= a.T) left = 0;  // an absent token of the tile
   const size_t at = ((size_t)tile * G + g) * kDigTile + n;
-  a.d.mask[at * 16 + i] = (unsigned char)left;
-  if (left) {
-#pragma unroll
-    for (int e = 0; e < 8; e++)
-      if (left >> e & 1) a.d.out[(size_t)t * a.cols + col + e] = v[e];
-  }
   const unsigned some = (unsigned)(__ballot(left != 0) >> (lane & 48)) & 0xffffu;
+  if (some) a.d.mask[at * 16 + i] = (unsigned char)left;
   // int4 codes enter the MFMA as 16 * (nibble - 8)
   if (i == 0) {
     const float sc = mb == 0 ? 0.0f : __builtin_ldexpf(ROWS8 ? 1.0f : 0.0625f, -k);
@@ -195,8 +197,9 @@ __global__ __launch_bounds__(64) void k_mix_digits(DigitArgs a) {
 // The columns of one token and group that are outside the digits: their
 // products with the codes of this lane's four rows, code(e, column).
 template <class Code>
-__device__ __forceinline__ void add_left_out(const unsigned char *mask, const float *out, const v4f &s4, v4f &acc,
-                                             Code code) {
+__device__ __forceinline__ void add_left_out(const float *asc, const unsigned char *mask, const float *out, const v4f &s4,
+                                             v4f &acc, Code code) {
+  if (!(__float_as_uint(*asc) >> 31)) return;
   const uint4 m = *(const uint4 *)mask;
   const unsigned w[4] = {m.x, m.y, m.z, m.w};
 #pragma unroll 1
@@ -442,7 +445,8 @@ __global__ __launch_bounds__(64 * W) void k_mix_mfma(MfmaArgs a) {
       int l = lane;
       asm volatile("" : "+v"(l));  // addresses formed here, not held in registers through the launch
       const int ln = l & 15, row = 4 * (l >> 4), tok = ln < nt ? ln : 0;
-      add_left_out(a.d.mask + (((size_t)blockIdx.y * a.G + g0 + j) * kDigTile + tok) * 16,
+      const size_t at = ((size_t)blockIdx.y * a.G + g0 + j) * kDigTile + tok;
+      add_left_out(a.d.asc + at, a.d.mask + at * 16,
                    a.d.out + ((size_t)(t0 + tok) * a.G + g0 + j) * 128,
                    FMT == 4 ? *(const v4f *)(sc + 16 * j + row) : v4f{1.f, 1.f, 1.f, 1.f}, acc, [&](int e, int c) {
                      const int at = FMT == 4 ? j * 1024 + ((c & 31) >> 1) : (2 * j + (c >> 4 & 1)) * 1024 + (c & 15);
@@ -627,7 +631,8 @@ __global__ __launch_bounds__(512) void k_mix_gemm(MfmaArgs a) {
           q[e] = pm.q + (size_t)rc * pm.rb + (size_t)g * (FMT == 4 ? 64 : 128);
           s4[e] = FMT == 4 ? pm.s[(size_t)rc * pm.ng + g] : 1.0f;
         }
-        add_left_out(a.d.mask + (((size_t)tt * a.G + g) * kDigTile + n) * 16,
+        const size_t at = ((size_t)tt * a.G + g) * kDigTile + n;
+        add_left_out(a.d.asc + at, a.d.mask + at * 16,
                      a.d.out + ((size_t)(t < a.T ? t : 0) * a.G + g) * 128, s4, acc[r][j],
                      [&](int e, int c) { return code_of<FMT>(q[e][FMT == 4 ? c >> 1 : c], c); });
       }
