@@ -145,7 +145,7 @@ __global__ __launch_bounds__(64) void k_mix_digits(DigitArgs a) {
 #pragma unroll
     for (int e = 0; e < 8; e++) cnt += (__float_as_uint(v[e]) & 0x7fffffffu) >= lo;
     bool drop = mb != 0 && (row_sum_i32(cnt) < kDigBulk || bad || tiny);
-    if (__ballot(drop) == 0) break;
+    if (__builtin_expect(__ballot(drop) == 0, 1)) break;
     bool lossy = bad || tiny;
 #pragma unroll
     for (int e = 0; e < 8; e++) {
@@ -186,7 +186,7 @@ __global__ __launch_bounds__(64) void k_mix_digits(DigitArgs a) {
     }
   const size_t at = ((size_t)tile * G + g) * kDigTile + n;
   const unsigned some = (unsigned)(__ballot(left != 0) >> (lane & 48)) & 0xffffu;
-  if (some) a.d.mask[at * 16 + i] = (unsigned char)left;
+  if (__builtin_expect(some != 0, 0)) a.d.mask[at * 16 + i] = (unsigned char)left;
   // int4 codes enter the MFMA as 16 * (nibble - 8)
   if (i == 0) {
     const float sc = mb == 0 ? 0.0f : __builtin_ldexpf(ROWS8 ? 1.0f : 0.0625f, -k);
@@ -440,7 +440,7 @@ __global__ __launch_bounds__(64 * W) void k_mix_mfma(MfmaArgs a) {
       }
     }
 #pragma unroll 1
-    for (unsigned u = left; u; u &= u - 1) {
+    for (unsigned u = left; __builtin_expect(u != 0, 0); u &= u - 1) {
       const int j = __builtin_ctz(u);
       int l = lane;
       asm volatile("" : "+v"(l));  // addresses formed here, not held in registers through the launch
@@ -619,7 +619,7 @@ __global__ __launch_bounds__(512) void k_mix_gemm(MfmaArgs a) {
   for (int j = 0; j < NTW; j++) {
     const int tl = tile0 + wn * NTW + j, tt = tl < ttiles ? tl : ttiles - 1, t = tt * kDigTile + n;
 #pragma unroll 1
-    for (unsigned long long u = left[j]; u; u &= u - 1) {
+    for (unsigned long long u = left[j]; __builtin_expect(u != 0, 0); u &= u - 1) {
       const int g = __builtin_ctzll(u);
 #pragma unroll
       for (int r = 0; r < RT; r++) {
