@@ -40,7 +40,8 @@ __global__ __launch_bounds__(256) void k_head_norm(signed char *xq, float *sx, f
   for (int i = threadIdx.x; i < np; i += blockDim.x) hp[i] = i < n ? xs[i] * xs[i] : 0.0f;
   __syncthreads();
   if (threadIdx.x < 64) {
-    const float ms = serial_sum_nonneg(hp, n, 0.0f);
+    // 6, 12: eight rows of 4,096 30.6 -> 29.6 us with 64 logits, 29.1 without a bound
+    const float ms = serial_sum_nonneg<6, 12>(hp, n, 0.0f);
     if (threadIdx.x == 0) s_r = 1.0f / sqrtf(ms / (float)n + eps);
   }
   __syncthreads();

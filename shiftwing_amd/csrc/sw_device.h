@@ -275,16 +275,17 @@ __device__ __forceinline__ float serial_sum_lds(const float *p, int m, float s =
 // large for exact scaling.  A run is about 750 cycles of dependent code, as
 // long as 57 dependent adds.  Squares of shorter mantissas (bf16 activations,
 // integers) tie far more often, growing rows change binade: a step with more
-// than kSerialTies tied lanes ahead of it, or kSerialRuns ended runs behind it,
-// adds its rest one by one, and after kSerialBad steps that left more than half
-// of themselves so, the row does.  A norm of 2,048 / 4,096 values by one lane's
+// than TIES tied lanes ahead of it, or RUNS ended runs behind it, adds its rest
+// one by one, and after kSerialBad steps that left more than half of themselves
+// so, the row does.  A norm of 2,048 / 4,096 values by one lane's
 // adds alone 12.1 / 22.7 us; this way 6.6 / 11.0 of full mantissas, 9.6 / 16.9 of
 // bf16 values (62 / 70 without the bound), 9.4 / 16.2 of nothing but ties (144 / 290).
 constexpr int kSerialStep = 512;
-constexpr int kSerialRuns = 4, kSerialTies = 6, kSerialBad = 2;
+constexpr int kSerialBad = 2;
 __device__ __forceinline__ float lane_value(float v, int l) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
 }
+template <int RUNS = 4, int TIES = 6>
 __device__ __forceinline__ float serial_sum_nonneg(const float *p, int m, float s) {
   const int lane = threadIdx.x & 63;
   const int mp = (m + 63) & ~63;
@@ -312,7 +313,7 @@ __device__ __forceinline__ float serial_sum_nonneg(const float *p, int m, float 
     if (__ballot(some) == 0) continue;
     bool plain = false;
     for (int runs = 0; l0 < 64 && !plain; runs++) {
-      if (runs == kSerialRuns) {
+      if (runs == RUNS) {
         plain = true;
         break;
       }
@@ -333,7 +334,7 @@ __device__ __forceinline__ float serial_sum_nonneg(const float *p, int m, float 
         }
         int sum = 0, ties = 0, at_tie = 0;
         const unsigned long long tied = __ballot(on && tie && !big);
-        if (__builtin_popcountll(tied) > kSerialTies) {
+        if (__builtin_popcountll(tied) > TIES) {
           plain = true;
           break;
         }

@@ -7,6 +7,8 @@ import time
 import numpy as np
 import pytest
 
+from test_gpu_output_head import _run
+
 pytestmark = pytest.mark.gpu
 
 
@@ -45,6 +47,21 @@ def test_ties_equal_the_chain(be, oracle, n):
     for b, name in enumerate(names):
         want = oracle.rmsnorm_zero(X[b], w, 1e-6)
         assert np.array_equal(got[b].view(np.uint32), want.view(np.uint32)), f"{name}, n={n}"
+
+
+@pytest.mark.parametrize("n", [576, 1000, 4096])
+def test_ties_equal_the_chain_in_the_output_head(be, oracle, n):
+    """The head's norm bounds its runs at other counts."""
+    rng = np.random.default_rng(n + 1)
+    names, rows = zip(*_rows(rng, n))
+    X = np.ascontiguousarray(np.stack([np.asarray(r, np.float32) for r in rows]))
+    w = (rng.standard_normal(n) * 0.1).astype(np.float32)
+    pad = (n + 15) // 16 * 16
+    q = rng.integers(-127, 128, (64, pad)).astype(np.int8)
+    hid, _ = _run(be, q, np.full(64, 1e-3, np.float32), X, w, 64, n, pad)
+    for b, name in enumerate(names):
+        want = oracle.rmsnorm_zero(X[b], w, 1e-6)
+        assert np.array_equal(hid[b].view(np.uint32), want.view(np.uint32)), f"{name}, n={n}"
 
 
 @pytest.mark.parametrize("n", [2048, 4096])
