@@ -537,7 +537,9 @@ int coli_cuda_moe_stack_trace(ColiCuda *ctx, unsigned long long *trace,
  * path's IDOT (qrow_i8(n), exact int32 dots, ((float)dot * scale) * sx;
  * c/qwen.c:1696-1705, 1765-1768).  Bit-exact with the CPU path.  `hidden`
  * (optional, [batch x cols]) receives n, which the reference also returns.
- * cols <= 16384; the matrix is streamed once per group of four rows. */
+ * cols <= 16384; the matrix is streamed once per 16 rows where they are
+ * aligned, have cols % 64 == 0 <= 8192 and are two or more (four above 2,048
+ * columns), else once per four rows. */
 int coli_cuda_output_head_q8(ColiCuda *ctx, float *logits, float *hidden,
                              const float *x, const float *norm_w, float eps,
                              int batch, const signed char *q,

@@ -244,7 +244,10 @@ extern "C" int coli_cuda_output_head_q8(ColiCuda *ctx, float *logits, float *hid
   const int nchp = nch <= 1 ? 1 : nch <= 2 ? 2 : nch <= 4 ? 4 : 8;
   // 1 / 2 / 4 / 8 tokens, MFMA against VALU dots: 2,048 columns 105 / 106 / 108 /
   // 114 against 95 / 115 / 154 / 293 us, 4,096 columns 210 / 211 / 215 / 224 against
-  // 165 / 189 / 278 / 534 (three tokens 113 against 105 at a vocabulary of 100,003)
+  // 165 / 189 / 278 / 534 (three tokens 113 against 105 at a vocabulary of 100,003).
+  // Vocabulary 151,936, two tokens at 512 / 1,024 / 1,536 columns 23 / 39 / 59 against
+  // 44 / 51 / 68, four at 2,560 / 3,072 / 5,120 / 8,192 99 / 111 / 192 / 263 against 144 /
+  // 150 / 243 / 355; three there take 110 / 117 / 205 / 288 by VALU dots
   if (fast && batch >= (cols <= 2048 ? 2 : 4) && cols % 64 == 0) {
     const int hl = head_cols(cols) * 16, cus = ctx->sm_count > 0 ? ctx->sm_count : 256;
     const hipError_t e = hipFuncSetAttribute((const void *)k_head_mfma, hipFuncAttributeMaxDynamicSharedMemorySize, hl);

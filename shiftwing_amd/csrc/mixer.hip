@@ -4,9 +4,9 @@
 //
 // What the reference computes (its CPU path, the contract): gdn_forward
 // c/qwen.c:3005-3030 with gdn_rule_step 2907-2927, gdn_decode_block 4642, and
-// attn_forward 3094-3137 with rope_head 3031.  Activations stay fp32 here
-// (the reference's GPU path rounds them to fp16 first); outputs agree with
-// the CPU path within 1e-3 x RMS.
+// attn_forward 3094-3137 with rope_head 3031.  Activations keep fp32's
+// precision here (the reference's GPU path rounds them to fp16 first); outputs
+// agree with the CPU path within 1e-3 x RMS.
 //
 // Gated DeltaNet step:
 //   projections            qkv and z of every token in one grid; whoever finishes

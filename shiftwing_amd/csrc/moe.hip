@@ -3347,8 +3347,11 @@ static void certify_launch(ColiCuda *ctx, ColiMoeLayer *L, Work &w, const float 
                                                                                        L->sgate_row);
 }
 
-// Blocks of 32 x 32 from which k_router_gemm<2> is the faster: 1,008 (1,999
-// tokens, S397) 185 against 276 us, 128 (512 tokens, S35) 35 against 24.
+// Blocks of 32 x 32 from which k_router_gemm<2> is the faster.  Routing by
+// 32 x 32 against 16 x 16 blocks at 128 / 192 / 256 / 320 / 384 / 448 / 512 / 1,024 of
+// them: S397 127 / 196 / 204 / 242 / 243 / 254 / 259 / 419 against 106 / 185 / 207 / 230 /
+// 247 / 276 / 289 / 504 us, S35 79 / 85 / 93 / 113 / 122 / 129 / 158 against 69 / 81 / 95 /
+// 108 / 124 / 140 / 174 (the blocks come in rounds of 256).
 constexpr int kRouterGemm2Blocks = 384;
 static int route_launch(ColiCuda *ctx, ColiMoeLayer *L, Work &w, const float *x) {
   hipStream_t st = ctx->stream;

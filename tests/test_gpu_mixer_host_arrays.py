@@ -129,4 +129,4 @@ def test_two_tokens_wait_for_no_copy_each(be):
             best = min(best, (time.perf_counter() - t) / 40 * 1e6)
         us.append(best)
     print(f"[host arrays] two tokens: device {us[0]:.1f}, host {us[1]:.1f} us", flush=True)
-    assert us[1] < 2.4 * us[0]
+    assert us[1] < 2.6 * us[0]

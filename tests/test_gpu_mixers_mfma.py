@@ -7,8 +7,10 @@ int8 output rows; against the oracle (or_gdn_forward / or_attn_forward).
 Tolerance: a projection of n <= 8192 products in fp32 is within n 2^-24
 sum|p| / RMS = 2^-24 n^1.5 of another order at worst and sqrt(n) of that in
 practice; with n = 512 here, and the layer's norms passing it on, 1e-4 x RMS
-leaves a factor of ten over the worst observed and is 10 times below what a
-wrong low digit (2^-8 of a value) would give."""
+leaves a factor of ten over the worst observed.  A wrong row, token or group
+shows at it, and a lost one of the two upper digits (up to 1 and 2^-7 of a
+group's largest value); the lower ones are test_gpu_mixer_precision.py's, which
+judges single projections against 64 bits."""
 import numpy as np
 import pytest
 
@@ -52,7 +54,8 @@ def test_gdn_projection_edges(be, oracle, H, kh, vh, dk, dv, K, slots, pos):
 
 @pytest.mark.parametrize("H,nh,nkv,o_fmt,rows", [(128, 2, 2, 4, 2), (128, 2, 1, 1, 15), (256, 4, 2, 4, 17),
                                                  (2304, 32, 2, 1, 33), (2304, 66, 6, 4, 16),
-                                                 # enough row and token tiles for the 128 x 128 blocks, both ragged
+                                                 # q, k, v in 128 x 128 blocks of one and two groups, both ragged;
+                                                 # o of 80 and 72 groups, which the vector kernels take
                                                  (256, 160, 10, 4, 401), (128, 144, 9, 1, 1025)])
 def test_gqa_projection_edges(be, oracle, H, nh, nkv, o_fmt, rows):
     from oracle import pyoracle as po
