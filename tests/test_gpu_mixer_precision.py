@@ -18,7 +18,7 @@ value) gives 1.9e-7."""
 import numpy as np
 import pytest
 
-from test_gpu_mixers import _dev_attn
+from test_gpu_mixers import _dev_attn, _dev_gdn
 
 pytestmark = pytest.mark.gpu
 CUS = 256
@@ -150,6 +150,22 @@ def test_wide_groups_prompt_chunk(be, kind):
     X = _wide(np.random.default_rng(108), kind, rows, 384)
     dev.prefill(X, 0)
     _check(dev.read_cache()[1][0], at.v, X, f"v, {kind}", _depth(384))
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("H,slots,pos", [(256, [0, 1, 2], [0, 5, 2]), (2048, [0, 0, 0, 0, 1], [0, 1, 2, 3, 0]),
+                                         (4224, list(range(16)), [7] * 16)])
+def test_wide_groups_in_the_convolution_ring(be, kind, H, slots, pos):
+    """The ring holds the qkv projection of each sequence's last tokens."""
+    from oracle import pyoracle as po
+    g = po.HostGdn(113, H, 1, 4, 32, 32)
+    dev = _dev_gdn(be, g, slots=max(slots) + 1)
+    X = _wide(np.random.default_rng(114), kind, len(slots), H)
+    zero = np.zeros((len(slots), 4), np.float32)
+    dev.slots_step(X, zero, zero, slots, pos, device_io=True)
+    ring = dev.read_state()[0]
+    raw = np.stack([ring[s, q % g.K] for s, q in zip(slots, pos)])
+    _check(raw, g.qkv, X, f"qkv, {kind}", _depth(H))
 
 
 def test_wide_groups_int8_prompt_chunk(be):
